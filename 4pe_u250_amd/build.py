@@ -42,7 +42,8 @@ HIP_FLAGS = [
     # preload nothing.
     "-mllvm", "-amdgpu-kernarg-preload-count=8",
 ]
-SOURCES = ["swiftkv_kernels.hip", "swiftkv_synth.hip", "swiftkv_exact.hip", "swiftkv_capi.cpp"]
+SOURCES = ["swiftkv_kernels.hip", "swiftkv_synth.hip", "swiftkv_exact.hip", "swiftkv_exact_short.hip",
+           "swiftkv_capi.cpp"]
 HOST_SRC = os.path.join(PKG_DIR, "host", "swiftkv_host.cpp")
 HOST_BIN = os.path.join(PKG_DIR, "swiftkv_host")
 

@@ -115,6 +115,10 @@ struct swiftkv_context {
     // launches that split no head: the step reads its arrival word on every
     // path but only a split head's merge writes one
     uint64_t* arrivals = nullptr;
+    // workspace of the integer-compatibility step: the exp2 table, then the
+    // split exchange (kExactWorkspaceWords; fixed, so a graph may record it at
+    // any time)
+    uint64_t* exact_workspace = nullptr;
     uint8_t* scratch = nullptr;     // this device's allocation-free workspace (arrival words, then partials)
     // Fault word of the split merges: pinned host memory that a step kernel
     // writes (system scope) when a merge gives up on a partial, read without
@@ -604,16 +608,25 @@ int run_step(swiftkv_context* ctx, const void* q, const void* k, const void* v, 
     return ok();
 }
 
-// Q30 exp2 table RNE(2^(30 + i/32)), i = 0..32 (swiftkv_attention.cpp:185-195).
-const uint32_t* exp2_table() {
-    static const std::vector<uint32_t> table = [] {
-        std::vector<uint32_t> t(33);
-        for (int i = 0; i < 33; ++i)
-            t[i] = static_cast<uint32_t>(std::nearbyint(std::ldexp(std::pow(2.0, i / 32.0), 30)));
-        return t;
-    }();
-    return table.data();
+// Tokens per split of the integer-compatibility step: whole quanta, at least
+// kExactMinSplit (one 64-token block per wave).
+constexpr int32_t kExactMinSplit = 256;
+int32_t exact_split(int32_t max_pos, int32_t batch) {
+    const int32_t len = max_pos + 1, splits = exact_splits(batch);
+    const int32_t tokens = std::max((len + splits - 1) / splits, kExactMinSplit);
+    return std::min((tokens + kSplitQuantum - 1) / kSplitQuantum * kSplitQuantum, kExactMaxTokens);
 }
+
+// Which kernel an integer-compatibility launch runs: batches past 8 rows whose
+// longest sequence is short take the one with four workgroups per CU (whose
+// turns hide each other's latencies), the rest the one that sums in any order
+// (one workgroup per CU).  Context 512 / 1024 / 2048, us, short kernel against
+// the other: batch 9 27.5 / 42.5 / 72.2 against 29.2 / 39.7 / 57.6; batch 16
+// 30.6 / 48.1 / 78.3 against 33.8 / 44.2 / 65.8; batch 24 35.4 / 57.0 / 97.9
+// against 45.0 / 59.7 / 92.5; batch 64 74.6 / 127.0 / 226.6 against 99.1 /
+// 135.6 / 217.0.  Up to 8 rows (one turn per workgroup) the other kernel is
+// ahead at every context.
+bool exact_is_short(int32_t max_pos, int32_t batch) { return batch > 8 && max_pos + 1 <= (batch <= 16 ? 768 : 1280); }
 
 int run_exact(swiftkv_context* ctx, const void* q, const void* k, const void* v, StepInput in,
               swiftkv_kv_cache* kv, const swiftkv_rope_lut* lut, uint8_t* act_q, uint8_t* act_scale,
@@ -641,8 +654,16 @@ int run_exact(swiftkv_context* ctx, const void* q, const void* k, const void* v,
         a.act_q = act_q ? act_q + static_cast<size_t>(b0) * kHeads * kGroupsPerHead * SWIFTKV_A14_WORD_BYTES
                         : nullptr;
         a.act_scale = act_scale ? act_scale + static_cast<size_t>(b0) * kHeads * kGroupsPerHead : nullptr;
+        int32_t max_pos = 0;
+        for (int32_t b = 0; b < nb; ++b) max_pos = std::max(max_pos, positions[b0 + b]);
+        a.split_tokens = exact_split(max_pos, nb);
+        const int32_t grid_splits = (max_pos + a.split_tokens) / a.split_tokens;
+        a.partials = ctx->exact_workspace;
+        a.merge_polls = ctx->merge_fault_test ? 1u : kMergePolls;
+        a.merge_tag_skew = ctx->merge_fault_test ? 1u : 0u;
         ProfilePair* p = profile_begin(ctx, SWIFTKV_KERNEL_EXACT);
-        SKV_HIP(launch_exact(a, exp2_table(), in.format == kInQ17, ctx->stream));
+        SKV_HIP(exact_is_short(max_pos, nb) ? launch_exact_short(a, in.format == kInQ17, ctx->stream)
+                                            : launch_exact(a, grid_splits, ctx->cus, in.format == kInQ17, ctx->stream));
         profile_end(ctx, p);
     }
     return ok();
@@ -728,6 +749,17 @@ float shift_to_scale(uint32_t s) {
     return f;
 }
 
+// Q30 exp2 table RNE(2^(30 + i/32)), i = 0..32 (swiftkv_attention.cpp:185-195).
+const uint32_t* exp2_table() {
+    static const std::vector<uint32_t> table = [] {
+        std::vector<uint32_t> t(33);
+        for (int i = 0; i < 33; ++i)
+            t[i] = static_cast<uint32_t>(std::nearbyint(std::ldexp(std::pow(2.0, i / 32.0), 30)));
+        return t;
+    }();
+    return table.data();
+}
+
 // Releases everything the context owns (after its last object is gone).
 void free_context(swiftkv_context* ctx) {
     (void)hipSetDevice(ctx->device);
@@ -735,6 +767,7 @@ void free_context(swiftkv_context* ctx) {
     if (ctx->partials) (void)hipFree(ctx->partials);
     for (void* p : ctx->retired) (void)hipFree(p);
     if (ctx->arrivals) (void)hipFree(ctx->arrivals);
+    if (ctx->exact_workspace) (void)hipFree(ctx->exact_workspace);
     if (ctx->io_stage) (void)hipFree(ctx->io_stage);
     if (ctx->fault_host) (void)hipHostFree(ctx->fault_host);
     for (auto& t : ctx->timers)
@@ -772,6 +805,10 @@ int swiftkv_context_create(int device, swiftkv_context** out) {
     const size_t arrival_bytes = sizeof(uint64_t) * kMaxBatchPerLaunch * kHeads * kArrivalStride;
     if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&ctx->arrivals), arrival_bytes);
     if (e == hipSuccess) e = hipMemset(ctx->arrivals, 0, arrival_bytes);
+    const size_t exact_bytes = sizeof(uint64_t) * kExactWorkspaceWords;
+    if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void**>(&ctx->exact_workspace), exact_bytes);
+    if (e == hipSuccess) e = hipMemset(ctx->exact_workspace, 0, exact_bytes);
+    if (e == hipSuccess) e = hipMemcpy(ctx->exact_workspace, exp2_table(), 33 * sizeof(uint32_t), hipMemcpyHostToDevice);
     void* scratch = nullptr;
     if (e == hipSuccess) e = scratch_for_device(device, count, ctx->stream, &scratch);
     ctx->scratch = static_cast<uint8_t*>(scratch);
@@ -895,6 +932,12 @@ int swiftkv_debug_set_split_generation(swiftkv_context* ctx, uint32_t generation
         base = ctx->partials;
         rows = ctx->partial_rows;
         slots = ctx->partial_slots;
+    }
+    if (!noalloc) {
+        uint64_t* const exact = ctx->exact_workspace + kExactTableWords;
+        SKV_HIP(launch_fill_u64(exact, kExactArrivalWords, static_cast<uint64_t>(generation) << 32, ctx->stream));
+        SKV_HIP(launch_fill_u64(exact + kExactArrivalWords, kExactWorkspaceWords - kExactTableWords - kExactArrivalWords,
+                                0, ctx->stream));
     }
     if (!base) return ok();   // no split workspace yet: the first one starts at generation 0
     const size_t arrivals = arrival_words(rows);

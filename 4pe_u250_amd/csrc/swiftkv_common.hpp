@@ -187,6 +187,39 @@ constexpr size_t kNoAllocPartialBytes =
     sizeof(uint64_t) * kNoAllocSplitRows * kHeads * kFixedSlots * kSlotWords;
 constexpr size_t kNoAllocScratchBytes = kNoAllocCounterBytes + kNoAllocPartialBytes;
 
+// Integer-compatibility step: positions stay below the reference's bound, so
+// one workgroup can hold a whole head's scores.  A CU holds one workgroup, and
+// launches whose heads leave CUs idle split each head up to exact_splits(batch)
+// ways (a multiple of 32 heads x splits up to 256).  The exchange workspace
+// reserves, for row b, the most splits a launch with that row has, so a slot
+// always belongs to the same (row, head, split).
+constexpr int kExactMaxTokens = 4096;
+constexpr int kExactMaxSplits = 8;
+constexpr int kExactSplitRows = 4;
+constexpr int kExactEntries = 9;                 // sums a split can publish: 8 after new maxima (or the new token)
+constexpr int kExactSlotWords = 64 + kExactEntries * 2 * kHeadDim;
+__host__ __device__ constexpr int exact_splits(int batch) { return batch > kExactSplitRows ? 1 : kExactMaxSplits / batch; }
+// Slots of row b and of the rows before it, a byte each (device code reads
+// them with one shift).
+__host__ __device__ constexpr int exact_row_slots(int b) { return (0x02020408u >> (8 * b)) & 0xff; }
+__host__ __device__ constexpr int exact_first_slot(int b) { return (0x0e0c0800u >> (8 * b)) & 0xff; }
+constexpr int kExactSlots = exact_first_slot(kExactSplitRows - 1) + exact_row_slots(kExactSplitRows - 1);
+constexpr bool exact_slot_tables_agree() {
+    for (int b = 0; b < kExactSplitRows; ++b)
+        if (exact_row_slots(b) != exact_splits(b + 1) ||
+            (b > 0 && exact_first_slot(b) != exact_first_slot(b - 1) + exact_row_slots(b - 1)))
+            return false;
+    return exact_first_slot(0) == 0;
+}
+static_assert(exact_slot_tables_agree(), "slot tables follow exact_splits");
+// The workspace: 64 words of 32 bits whose first 33 are the Q30 exp2 table
+// RNE(2^(30 + i/32)) (swiftkv_attention.cpp:185-195), the arrival words, the
+// slots; in 64-bit words.
+constexpr int kExactTableWords = 32;
+constexpr size_t kExactArrivalWords = static_cast<size_t>(kExactSplitRows) * kHeads * kArrivalStride;
+constexpr size_t kExactWorkspaceWords =
+    kExactTableWords + kExactArrivalWords + static_cast<size_t>(kExactSlots) * kHeads * kExactSlotWords;
+
 // Launchers (swiftkv_kernels.hip).
 // shape: one of SWIFTKV_STEP_SHAPES (hipErrorInvalidValue otherwise).
 hipError_t launch_step(const StepArgs& a, int grid_splits, StepShape shape, InputFormat in, hipStream_t s);
@@ -199,9 +232,14 @@ hipError_t launch_fill_u64(uint64_t* p, size_t n, uint64_t value, hipStream_t s)
 // Device address of the allocation-free workspace on the current device,
 // zero-filled by a kernel on `s` (waits for it).  Call once per device.
 hipError_t bind_noalloc_scratch(hipStream_t s, void** device_ptr);
-// Integer-compatibility step (one workgroup per (sequence, head)); a.out is
-// int32 Q15.17; exp_lut holds the 33 Q30 exp2 entries.
-hipError_t launch_exact(const StepArgs& a, const uint32_t* exp_lut, bool q17, hipStream_t s);
+// Integer-compatibility step on a device of `cus` compute units
+// (a.split_tokens tokens per workgroup when grid_splits > 1, else whole heads);
+// a.out is int32 Q15.17, a.partials the workspace above.
+hipError_t launch_exact(const StepArgs& a, int grid_splits, int cus, bool q17, hipStream_t s);
+// The same for batches of short sequences, one workgroup per (sequence, head).
+hipError_t launch_exact_short(const StepArgs& a, bool q17, hipStream_t s);
+// The packed leading arguments of a launch (swiftkv_kernels.hip).
+StepPreload step_preload(const StepArgs& a);
 // out[i] = Q15.17 of in[i] (parts = 1) or of the reduced split-K partials
 // in[i + p * part_stride] (parts = 2 or 4).
 hipError_t launch_convert(const float* in, int32_t parts, int64_t part_stride, int32_t* out, size_t n,

@@ -1,825 +1,1239 @@
 // swiftkv_exact.hip -- integer-compatibility step: the reference's Q15.17
 // single-pass recurrence evaluated exactly on the GPU, so the A14 words and
 // E8M0 codes equal the reference's bit for bit (swiftkv_attention.cpp:934-1880;
-// llama2_decoder_sw_emulator.cpp:633-711).  Slow by construction -- the
-// (max, Z, Y) recurrence is sequential per head -- and meant for bit-level
-// comparison with the FPGA / C model; the sequential chains bound it, not HBM.
+// llama2_decoder_sw_emulator.cpp:633-711).
 //
-// Grid (32 heads x SLICES, batch rows), 256 threads per (sequence, head,
-// slice of 128 / SLICES channels); SLICES is 4 for the smallest batches, 2
-// up to batch 8 and 1 otherwise.  Wave 0 first appends the new row like the fast step; then
-// tokens [0, position] are processed in chunks of kChunk:
-//   - the 4 waves issue all of the chunk's loads at once through one buffer
-//     resource (K codes and scales into registers, V codes straight into
-//     LDS), then compute the integer
-//     scores (lane = 16-channel half-group c of token row r; the per-half
-//     shift and the 44-bit wraps are associative modulo 2^44, so the octet
-//     sum may run in any order), the exact 64-bit dot taken as signed-byte
-//     dot products over five limbs of the query;
-//   - one thread per token turns its score and the exclusive prefix maximum
-//     into a coefficient word (exp LUT, rescale flag), and the same pass lays
-//     out, per group, the product of the coefficient and the V scale (exact
-//     in FP32), the per-wave coefficient sums and ballots for Z and Y;
-//   - Y, one channel per thread: the first kCh threads run the chunk's
-//     first part in token order, adding independently formed terms, while
-//     the rest of the threads compose the remaining tokens (no first or
-//     rescaling token among them) into clamp-add maps applied after the
-//     barrier; a term is one fused multiply-add of the code and the product
-//     when the shift is at most 15, an exact FP32 product and rint at 16,
-//     32-bit integer operations above; wave 3 also advances Z by prefix-sum
-//     differences and steps only at first and rescaling tokens;
-// then Y * 1/Z and the integer-path A14/E8M0 epilogue.
-#include <type_traits>
+// The recurrence over (max, Z, Y) looks sequential, but only the tokens that
+// raise the running maximum (about ln n of n) must be taken in order:
+//   - the running maximum before a token is the prefix maximum of the scores,
+//     so all scores come first, then every coefficient at once;
+//   - an ordinary token adds a term to Y and its coefficient to Z that depend
+//     on neither; while no partial sum of Y can reach an end of the int32 range
+//     the saturating adds are plain adds, and a sum modulo 2^32 in any order is
+//     the reference's.  Each sum carries a bound of its terms' magnitudes; where
+//     |Y| plus the bound could reach 2^31 the segment is run token by token.
+//
+// One 8-wave workgroup per CU.  Launches that split heads have the grid
+// (splits, 32 heads, batch rows); workgroup (j, h, z) owns tokens [j*C,
+// min((j+1)*C, position)) of head h of rows[z]'s sequence.  The others have up
+// to one workgroup per CU, each taking whole heads in turn.  Per head:
+//   1. every wave loads its first K and V blocks (64 tokens: lane = chunk c =
+//      lane&7 of 16 channels, row r = lane>>3 of 8 rows), then rotates the
+//      query and splits it into signed-byte limbs; the last wave also quantizes
+//      the new row and scores it (the owner of `position` appends it);
+//   2. K pass: scores of the wave's blocks (round-robin) into LDS, with each
+//      block's maximum and the V scales' exponents;
+//   3. the block maxima are exchanged (LDS barrier; with several splits, one
+//      tagged word per split): the running maximum before every block, and which
+//      blocks hold a new one ("hot": usually three or four beyond the first);
+//   4. V pass: coefficients of the wave's blocks, then V codes straight from
+//      memory times coefficient times scale, rounded per term, summed per lane.
+//      A wave's sums go to LDS where a stretch between hot blocks ends; of a hot
+//      block, the tokens from its first to its last new maximum are left to 5,
+//      as terms in LDS;
+//   5. Y is folded over those few sums and terms in token order by one thread
+//      per channel, Z by one wave; the new token is the last step, then Y * 1/Z
+//      and the integer-path A14/E8M0 epilogue.
+// The next head's first blocks are loaded behind the last ones of this head, so
+// that the fold and the prologue run under them.
+//
+// With several splits, each publishes its sums and new maxima as tagged words,
+// and the last of a head to arrive folds them (the fast step's exchange).  A
+// split that cannot publish in full -- it did not hear of the maxima before it
+// in time, or has too many new ones -- says so, and then, or where a bound
+// fails, the last to arrive runs the whole head by itself: no wait is
+// unbounded and no result depends on who waits for whom.
+//
+// What bounds it: for small batches the chain of round trips (first loads 3 us,
+// K pass 3, exchange of maxima 1.3, V pass 3.5, fold 1-4, exchange of sums 3);
+// for large ones the stream, at 6.9 TB/s within the K and V passes of a head,
+// with about 7 us of fold, barriers and ramps per 50 us head.  Context 4096,
+// us per call, the chunked kernel it replaced (Y in token order through LDS, up
+// to four workgroups per head each scoring every token) against this one: batch
+// 1 88.7 / 25.0, 2 92.2 / 30.6, 4 89.3 / 40.4, 8 111.8 / 58.8, 16 135.2 / 112.3,
+// 64 429.6 / 391.4; context 1536 at batch 5 52.1 / 27.5.  Tried: two 8-wave
+// workgroups per CU (128 registers, 480 at batch 64: their streams get in each
+// other's way, and a batch-1 launch then doubles workgroups up on half the CUs,
+// 39 against 28); reloading each row as soon as it is used (426 against 431, but
+// the compiler gives the rows other registers in each loop and waits for all
+// loads to copy them); sums per piece between new maxima (a masked pass and a
+// reduction each, 5-6 us per head more).  Only a head whose every token is a new
+// maximum is slower than before (batch 32: 1992 against 538): its hot blocks
+// outrun the staging rows and run from the page in order.
+#include <algorithm>
 
-#include "swiftkv_device.hpp"
+#include "swiftkv_exact.hpp"
 
 namespace swiftkv {
 namespace {
 
-using namespace dev;
+using namespace exact;
 
-constexpr int kChunk = 256;                   // cached tokens per chunk (V codes staged in LDS)
-constexpr int kBatch = 8;                     // tokens whose LDS reads go out together in the Y pass
-static_assert(kChunk % kBatch == 0, "batches tile a chunk");
-static_assert(kBatch % 4 == 0 && 64 % kBatch == 0, "a batch is whole 16-byte reads inside one 64-token ballot");
-constexpr int kPasses = kChunk / 32;          // score passes per chunk: 4 waves x 8 token rows each
-// Largest batch whose launch splits each head's Y over 4 workgroups (32
-// channels each): at context 4096 this took batch 1 and 2 from 175 to 147-150
-// us, was even at batch 4 and slower from batch 8 on, where one workgroup per
-// head already fills the machine and the 4x score work shows.
-constexpr int kExactSlicedMaxBatch = 2;
-// Largest batch whose launch splits each head's Y over 2 workgroups (64
-// channels each): batch 3 and 4 ran 16-21% faster than with one workgroup
-// per head (whose 128 workgroups leave half the CUs idle), batch 6 and 8 up
-// to 6%; from batch 12 on the doubled score work made it slower.
-constexpr int kExactHalfSlicedMaxBatch = 8;
-constexpr int64_t kScoreScaleQ17 = 11585;     // RNE(2^17 / sqrt(128)) (swiftkv_attention.cpp:1101-1102)
-constexpr int64_t kLog2eQ21 = 3025551;        // RNE(log2(e) * 2^21) (cpp:207-208)
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * 64;
+constexpr int kBlock = 64;                    // tokens a wave takes at a time
+constexpr int kRows = kBlock / 8;             // token rows per lane of a block
+constexpr int kMaxBlocks = kExactMaxTokens / kBlock;
+static_assert(kMaxBlocks <= 64, "one lane per block where the block maxima are scanned");
+// Accumulators per workgroup: one per stretch between hot blocks and cuts (up
+// to 65), and in a split that cannot fold its own sums one per special token,
+// from the back.  4096 tokens in random order hold 8.9 +- 2.8 new maxima in
+// about five hot blocks.
+constexpr int kPool = 65 + kExactEntries - 1;
+constexpr int kSpecials = kExactEntries - 1;
+constexpr int kStageRows = 128;               // tokens of hot blocks staged in LDS
 
-__device__ __forceinline__ int64_t wrap_bits(int64_t x, int bits) {
-    const uint64_t mask = (1ull << bits) - 1u;
-    uint64_t r = static_cast<uint64_t>(x) & mask;
-    if ((r >> (bits - 1)) & 1u) r |= ~mask;
-    return static_cast<int64_t>(r);
-}
-
-// Round-half-even of x / 2^s (AP_RND_CONV), 1 <= s <= 31.  With q =
-// floor(x / 2^s) and r = x - q 2^s: r < 2^(s-1) gives q, r > 2^(s-1) gives
-// q + 1, and the tie gives q + (q & 1) -- all three are floor((x + 2^(s-1) - 1
-// + (q & 1)) / 2^s), for either sign of x.  RNE of the exact quotient is odd-
-// symmetric, so this equals rounding the magnitude and restoring the sign.
-__device__ __forceinline__ int64_t rne_shift(int64_t x, int s) {
-    return (x + ((int64_t{1} << (s - 1)) - 1) + ((x >> s) & 1)) >> s;
-}
-
-// Q15.17 x unsigned Q1.17 multiplier, RNE >> 17, wrapped to 32 bits.
-__device__ __forceinline__ int32_t mulq17_wrap(int32_t a, uint32_t b) {
-    return static_cast<int32_t>(static_cast<uint32_t>(
-        rne_shift(static_cast<int64_t>(a) * static_cast<int64_t>(b), 17)));   // low 32 bits = the wrap
-}
-
-// exp(x) for x <= 0 in Q1.17 through the 33-entry Q30 exp2 table with 12-bit
-// linear interpolation (swiftkv_attention.cpp:185-260).
-__device__ __forceinline__ uint32_t exp_neg_q17(int32_t x, const uint32_t* lut) {
-    if (x >= 0) return 1u << 17;
-    if (x <= -(32 << 17)) return 0u;
-    const int64_t l = wrap_bits(rne_shift(static_cast<int64_t>(x) * kLog2eQ21, 21), 24);
-    const int64_t ex = l >> 17;
-    const uint32_t f = static_cast<uint32_t>(l - (ex << 17));
-    const uint32_t idx = f >> 12, rm = f & 0xfffu;
-    const uint32_t base = lut[idx], next = lut[idx + 1];
-    const uint32_t interp = base + static_cast<uint32_t>((static_cast<uint64_t>(next - base) * rm + (1u << 11)) >> 12);
-    const int sh = 13 - static_cast<int>(ex);
-    uint64_t out = 0;
-    if (sh <= 0) out = static_cast<uint64_t>(interp) << (-sh);
-    else if (sh < 32) out = (static_cast<uint64_t>(interp) + (1ull << (sh - 1))) >> sh;
-    return static_cast<uint32_t>(out) & 0x3ffffu;
-}
-
-// The 16 rotated query channels of one half-group as five planes of signed
-// bytes, four channels per word: q = l0 + l1 2^8 + l2 2^16 + l3 2^24 + l4 2^32,
-// each limb the signed low byte of what the limbs below it leave, so every
-// limb lies in [-128, 127] and the top one in {-1, 0, 1} for any int32 q.
+// 16 rotated query channels as signed-byte limbs, q = l0 + l1 2^8 + l2 2^16 +
+// l3 2^24 + l4 2^32 (each limb in [-128, 127]): a lane holds limbs 0-2 of its
+// chunk's channels, four to a word; limbs 3 and 4 stay in LDS, as they are zero
+// for |q| below about 64.0.
 struct QueryLimbs {
-    int32_t w[5][4];
+    int32_t w[3][4];
 };
 
-__device__ __forceinline__ QueryLimbs split_query(const int32_t* q) {
-    QueryLimbs L;
+// Exact dot of 16 codes with limbs 0-2 of the query (|sum| < 2^35).
+__device__ __forceinline__ double limb_dot3(const QueryLimbs& L, v4i k) {
+    int32_t s[3];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        uint32_t packed[5] = {0u, 0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int byte = 0; byte < 4; ++byte) {
-            int64_t rest = q[4 * j + byte];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) {
-                const int32_t limb = static_cast<int8_t>(static_cast<uint8_t>(rest));
-                packed[k] |= static_cast<uint32_t>(static_cast<uint8_t>(limb)) << (8 * byte);
-                rest = (rest - limb) >> 8;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 5; ++k) L.w[k][j] = static_cast<int32_t>(packed[k]);
-    }
-    return L;
-}
-
-// 44-bit token dot contribution of one 16-channel half-group: the 16 int8
-// codes times the int32 rotated query, scaled by 2^(shift-10) (cpp:934-995).
-// The exact sum is taken limb by limb: four signed-byte dot products per limb
-// (each limb's sum stays within 16 * 128 * 128 = 2^18), then combined in 64
-// bits, so it equals the sum of the 16 full products.
-// NL = 3 when the wave's query limbs 3 and 4 are all zero (|q| below about
-// 2^23, i.e. |q| < 64.0, the common case): those limbs add nothing.
-template <int NL>
-__device__ __forceinline__ int64_t half_dot(const QueryLimbs& L, int4 w, uint32_t shift) {
-    const int32_t d[4] = {w.x, w.y, w.z, w.w};
-    int64_t s = 0;
-#pragma unroll
-    for (int k = NL - 1; k >= 0; --k) {
+    for (int i = 0; i < 3; ++i) {
         int32_t acc = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_sdot4(L.w[k][j], d[j], acc, false);
-        s = s * 256 + acc;
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_sdot4(L.w[i][j], k[j], acc, false);
+        s[i] = acc;
     }
-    const int64_t p = shift >= 10 ? static_cast<int64_t>(static_cast<uint64_t>(s) << (shift - 10))
-                                  : (s >> (10 - shift));
-    return wrap_bits(p, 44);
+    return __builtin_fma(static_cast<double>(s[2]), 65536.0, static_cast<double>(s[0] + s[1] * 256));
 }
 
-__device__ __forceinline__ int32_t score_of(int64_t token_dot) {
-    return sat32(rne_shift(wrap_bits(token_dot, 44) * kScoreScaleQ17, 24));
+__device__ __forceinline__ double octet_sum_f64(double x) {
+    x += __builtin_bit_cast(double, dpp64<kDppQuadXor1>(__builtin_bit_cast(int64_t, x)));
+    x += __builtin_bit_cast(double, dpp64<kDppQuadXor2>(__builtin_bit_cast(int64_t, x)));
+    return x + __builtin_bit_cast(double, dpp64<kDppHalfMirror>(__builtin_bit_cast(int64_t, x)));
 }
 
-__device__ __forceinline__ uint32_t shift_of(float scale) { return (__float_as_uint(scale) >> 23) - 110u; }
-
-// The single-pass recurrence (cpp:1276-1335, 1463-1558) in three parts.
-// The running maximum before token i is the prefix maximum of the scores
-// (the reference raises it only on a strictly larger score, and a maximum
-// does not depend on order), so every token's coefficient and rescale flag
-// follow from its score and that prefix maximum, for all tokens of a chunk at
-// once.  What stays sequential is Z at first and rescaling tokens, and Y.
-constexpr uint32_t kInit = 1u << 31;      // first token of the sequence: Y = v, Z = 1
-constexpr uint32_t kRescale = 1u << 30;   // new maximum: Y = Y * coef + v, Z = Z * coef + 1
-constexpr uint32_t kCoefMask = (1u << 18) - 1u;
-constexpr uint32_t kMask30 = (1u << 30) - 1u;
-
-// Coefficient word of a token with score s and prefix maximum `before`.
-__device__ __forceinline__ uint32_t coef_word(int32_t s, int32_t before, const uint32_t* lut) {
-    if (s <= before) return exp_neg_q17(sat32(static_cast<int64_t>(s) - before), lut);
-    return exp_neg_q17(sat32(static_cast<int64_t>(before) - s), lut) | kRescale;
+// Orders a wave's LDS writes before its own later reads of what other lanes
+// wrote (the hardware runs a wave's LDS operations in order).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Z in Q13.17, wrapped to 30 bits.
-__device__ __forceinline__ uint32_t z_step(uint32_t z, uint32_t word) {
-    if (word & kInit) return 1u << 17;
-    const uint32_t coef = word & kCoefMask;
-    if (word & kRescale)
-        return ((static_cast<uint32_t>(rne_shift(static_cast<int64_t>(z) * coef, 17)) & kMask30) + (1u << 17)) &
-               kMask30;
-    return (z + coef) & kMask30;
+// A wave-uniform value the compiler cannot see is uniform (it came through LDS
+// or memory), moved to a scalar register: control flow and buffer offsets that
+// depend on it stay scalar.
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
-// Y per token and channel (cpp:1463-1558):
-//   first token  Y = v
-//   no rescale   Y = sat32(Y + wrap32(RNE(v c >> 17)))
-//   rescale      Y = sat32(wrap32(RNE(Y c >> 17)) + v)
-// with v = code << shift as the reference's ap_int<32> (it wraps for code 64,
-// shift 25).  The no-rescale term does not depend on Y, so the terms of a
-// batch of tokens are formed independently and only the saturating adds run
-// in series.  The term in 32-bit operations, c < 2^18 and |code| <= 128:
-//   shift >= 17: v is a multiple of 2^17, so the quotient is exact and equals
-//                (v >> 17) c, with |v >> 17| <= 2^14 -- the low 32 bits of a
-//                24-bit product are the wrap;
-//   shift < 17:  v c = (code c) 2^shift exactly, |code c| < 2^25, so the term
-//                is RNE((code c) / 2^k) for k = 17 - shift in 1..17, in the
-//                floor((x + 2^(k-1) - 1 + bit k of x) >> k) form of rne_shift.
-__device__ __forceinline__ int32_t dequant_raw(int32_t code, uint32_t shift) {
-    return static_cast<int32_t>(static_cast<uint32_t>(code) << shift);
-}
+// ---------------------------------------------------------------- state
 
-// Both cases in one form: x = v >> min(shift, 17) is the code itself below
-// 17 and v >> 17 above, m = x c, and the rounding shift k = 17 - shift
-// clamps to 0 above 17, where the rounding terms (2^(16-shift) - 1 and a
-// zero-width bit field) vanish and the term is m.
-__device__ __forceinline__ int32_t value_term(int32_t code, uint32_t shift, uint32_t coef) {
-    const int32_t m = __mul24(dequant_raw(code, shift) >> min(shift, 17u), static_cast<int32_t>(coef));
-    const uint32_t k = __builtin_elementwise_sub_sat(17u, shift);
-    const int32_t bit = static_cast<int32_t>(__builtin_amdgcn_ubfe(static_cast<uint32_t>(m), k, min(k, 1u)));
-    return (m + static_cast<int32_t>(0xffffu >> shift) + bit) >> k;
-}
-
-__device__ __forceinline__ int32_t value_step(int32_t y, uint32_t word, int32_t code, uint32_t shift, int32_t term) {
-    if (word & kInit) return dequant_raw(code, shift);
-    if (word & kRescale) return __builtin_elementwise_add_sat(mulq17_wrap(y, word & kCoefMask), dequant_raw(code, shift));
-    return __builtin_elementwise_add_sat(y, term);
-}
-
-
-// Sum over the 8 lanes of an aligned octet of a 64-bit integer (DPP moves of
-// both halves, integer adds, so exact in any order); every lane gets it.
-template <int Ctrl>
-__device__ __forceinline__ int64_t dpp64(int64_t x) {
-    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), Ctrl, 0xF, 0xF, true));
-    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x >> 32), Ctrl, 0xF, 0xF, true));
-    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
-}
-__device__ __forceinline__ int64_t octet_sum64(int64_t x) {
-    x += dpp64<kDppQuadXor1>(x);
-    x += dpp64<kDppQuadXor2>(x);
-    return x + dpp64<kDppHalfMirror>(x);
-}
-
-// Inclusive wave scans with DPP (GFX9): row shifts by 1, 2, 4, 8 scan each
-// 16-lane row, then row 0's last lane is broadcast into row 1 and row 2's
-// into row 3, then lane 31 into rows 2 and 3.  Lanes a move cannot reach, and
-// rows outside its row mask, take the identity.
-constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114, kDppRowShr8 = 0x118;
-constexpr int kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143, kDppWaveShr1 = 0x138;
-
-template <int Ctrl, int RowMask>
-__device__ __forceinline__ int32_t dpp_shifted(int32_t identity, int32_t x) {
-    return __builtin_amdgcn_update_dpp(identity, x, Ctrl, RowMask, 0xF, false);
-}
-
-__device__ __forceinline__ int32_t wave_scan_max(int32_t x) {
-    x = max(x, dpp_shifted<kDppRowShr1, 0xF>(INT32_MIN, x));
-    x = max(x, dpp_shifted<kDppRowShr2, 0xF>(INT32_MIN, x));
-    x = max(x, dpp_shifted<kDppRowShr4, 0xF>(INT32_MIN, x));
-    x = max(x, dpp_shifted<kDppRowShr8, 0xF>(INT32_MIN, x));
-    x = max(x, dpp_shifted<kDppRowBcast15, 0xA>(INT32_MIN, x));
-    return max(x, dpp_shifted<kDppRowBcast31, 0xC>(INT32_MIN, x));
-}
-
-__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
-    int32_t x = static_cast<int32_t>(v);
-    x += dpp_shifted<kDppRowShr1, 0xF>(0, x);
-    x += dpp_shifted<kDppRowShr2, 0xF>(0, x);
-    x += dpp_shifted<kDppRowShr4, 0xF>(0, x);
-    x += dpp_shifted<kDppRowShr8, 0xF>(0, x);
-    x += dpp_shifted<kDppRowBcast15, 0xA>(0, x);
-    return static_cast<uint32_t>(x + dpp_shifted<kDppRowBcast31, 0xC>(0, x));
-}
-
-// A wave-uniform 64-bit value read by every lane, moved to scalar registers.
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    return (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v >> 32))))
-            << 32) |
-           static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
-}
-
-// The Y pass reads, per token and G32 group, the product p = c 2^(s-17) of
-// the token's coefficient c (an integer, at most 2^17) and the group's V
-// scale 2^(s-17); the FP32 product is exact.  The no-rescale term is then
-// RNE(code p), since v c 2^-17 = (code 2^s) c 2^-17 for a shift below 17.
-//
-// Shift at most 15 (V groups below 32.0, the common case): |code p| <= 128
-// 2^15 = 2^22, so code p + 1.5 2^23 lies in [2^23, 2^24), where the floats
-// are the integers.  One fused multiply-add rounds the exact sum once, to
-// nearest even, and 1.5 2^23 is an even integer, so the result is 1.5 2^23 +
-// RNE(code p) and its bit pattern is 0x4b400000 + RNE(code p).
-constexpr float kRoundMagic = 12582912.0f;   // 1.5 * 2^23
-constexpr uint32_t kRoundMagicBits = 0x4b400000u;
-__device__ __forceinline__ uint32_t term_bits(int32_t code, float p) {
-    return __float_as_uint(__builtin_fmaf(static_cast<float>(code), p, kRoundMagic));
-}
-// A term of that form is at most 2^22 in magnitude.
-constexpr int64_t kFastTermBound = int64_t{1} << 22;
-
-// The codes and Y terms of tokens [i0, i0 + kBatch) for channel ch, for any
-// shift: the coefficient words come from 16-byte reads, the products p of the
-// channel's group from 16-byte reads, the codes from one byte read per token.
-// A first or rescaling token's p is its V scale alone (its term is not used).
-// wide17: some token of the batch has a shift of 17 or more.  Otherwise every
-// |code c| <= 2^24 is exact in FP32, so code p is exact and rint gives RNE
-// (the short form, returns true); else the shift is recovered from the
-// exponents of p and c and the 32-bit integer form runs (returns false).
-__device__ __forceinline__ bool slow_terms(const uint32_t* s_words, const float* s_p_g,
-                                           const int8_t (*s_vc)[kHeadDim], int i0, int ch, bool wide17,
-                                           int32_t* code, float* p, int32_t* term) {
-    uint32_t coef[kBatch];
-#pragma unroll
-    for (int q = 0; q < kBatch / 4; ++q) {
-        const uint4 cq = *reinterpret_cast<const uint4*>(&s_words[i0 + 4 * q]);
-        const float4 pq = *reinterpret_cast<const float4*>(&s_p_g[i0 + 4 * q]);
-        coef[4 * q] = cq.x & kCoefMask;
-        coef[4 * q + 1] = cq.y & kCoefMask;
-        coef[4 * q + 2] = cq.z & kCoefMask;
-        coef[4 * q + 3] = cq.w & kCoefMask;
-        p[4 * q] = pq.x;
-        p[4 * q + 1] = pq.y;
-        p[4 * q + 2] = pq.z;
-        p[4 * q + 3] = pq.w;
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) code[j] = s_vc[i0 + j][ch];
-    if (!wide17) {
-#pragma unroll
-        for (int j = 0; j < kBatch; ++j) term[j] = static_cast<int32_t>(__builtin_rintf(static_cast<float>(code[j]) * p[j]));
-        return true;
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-        // p = c 2^(s-17) exactly, so s = 17 + exponent(p) - exponent(c); a
-        // zero coefficient gives a zero term for any shift.
-        const uint32_t sh = coef[j] == 0u ? 0u
-                                          : min(17u + shift_of(p[j]) - shift_of(static_cast<float>(coef[j])), 25u);
-        term[j] = value_term(code[j], sh, coef[j]);
-    }
-    return false;
-}
-// A short-form term is at most 128 2^16 = 2^23 in magnitude.
-constexpr int64_t kShortTermBound = int64_t{1} << 23;
-
-// What the fused-multiply-add terms of tokens [i0, i0 + kBatch) for channel
-// ch read: the products p of the channel's group and the codes.
-struct FastBatch {
-    float p[kBatch];
-    int32_t code[kBatch];
-};
-__device__ __forceinline__ FastBatch load_fast(const float* s_p_g, const int8_t (*s_vc)[kHeadDim], int i0, int ch) {
-    FastBatch f;
-#pragma unroll
-    for (int q = 0; q < kBatch / 4; ++q) {
-        const float4 pq = *reinterpret_cast<const float4*>(&s_p_g[i0 + 4 * q]);
-        f.p[4 * q] = pq.x;
-        f.p[4 * q + 1] = pq.y;
-        f.p[4 * q + 2] = pq.z;
-        f.p[4 * q + 3] = pq.w;
-    }
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) f.code[j] = s_vc[i0 + j][ch];
-    return f;
-}
-// The term bits 0x4b400000 + term of such a batch, every shift at most 15.
-__device__ __forceinline__ void fast_term_bits(const FastBatch& f, uint32_t* tb) {
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) tb[j] = term_bits(f.code[j], f.p[j]);
-}
-constexpr uint64_t kBatchMask = (uint64_t{1} << kBatch) - 1u;
-// No partial sum of a batch of fused-multiply-add terms exceeds this.
-constexpr uint32_t kSatMargin = static_cast<uint32_t>(kBatch * kFastTermBound);
-
-// The per-group products p of a chunk and the query's LDS bytes: shared
-// with one workgroup per head (where LDS bounds the residency: four
-// workgroups per CU), separate with four (three per CU by registers).
-template <int G, int CH>
-union ProductsOrQuery {
-    float p[G][kChunk];
-    int32_t q[kHeadDim];
-    int16_t q14[CH];
-};
-template <int G, int CH>
-struct ProductsAndQuery {
-    float p[G][kChunk];
-    int32_t q[kHeadDim];
-    int16_t q14[CH];
+struct Shared {
+    // Per token of the range: x is the score, then the coefficient as a float
+    // (sign set for a first or rescaling token, zero past the range); y the
+    // biased exponents of the token's four V scales, a byte each.
+    uint2 tok[kExactMaxTokens];
+    // Sums of ordinary terms, modulo 2^32, of the coefficients, and of
+    // coefficient times scale per group (the bound).
+    int32_t pool[kPool][kHeadDim];
+    uint32_t pool_z[kPool];
+    float pool_b[kPool][kGroupsPerHead];
+    // Folding workgroups, per hot block: its tokens from the first to the last
+    // special one, {first token | past the last << 16, row of `stage` where
+    // they start (not staged if they would end past it), what Y is multiplied
+    // by at the first}; per staged token what Y is multiplied by (1.0 for an
+    // ordinary one) and what is added.
+    uint4 hot[kPool];
+    uint32_t stage_mult[kStageRows];
+    int32_t stage[kStageRows][kHeadDim];
+    uint32_t staged;                              // rows taken so far
+    // Special (first or rescaling) tokens of a split that cannot fold its own
+    // sums; number i uses pool entry kPool-1-i for the ordinary tokens after
+    // it in its block.  Per hot block: its first special token and their count.
+    int8_t code[kSpecials][kHeadDim];
+    uint32_t sp_word[kSpecials];
+    uint32_t sp_exps[kSpecials];
+    uint32_t hot_first[kPool];
+    uint32_t hot_count[kPool];
+    int32_t blk_max[kMaxBlocks];                  // per block: its largest score
+    int32_t blk_exp[kMaxBlocks];                  // and the largest biased exponent of its V scales
+    uint32_t limb_hi[2][kHeadDim / 4];            // query limbs 3 and 4
+    uint32_t lut[33];
+    int8_t new_code[kHeadDim];                    // the new token
+    uint32_t new_exps;
+    int32_t new_score;
+    uint32_t specials;                            // special tokens so far
+    int32_t prefix;                               // running maximum before the range
+    uint32_t failed;                              // the range's sums are incomplete
+    uint32_t z;                                   // Z over the range
+    uint32_t new_word;                            // the new token's coefficient word
+    uint32_t redo;                                // the splits' sums cannot be used
+    uint32_t last;
+    uint32_t misc[16];                            // the split's own count and words of entries 0 and 1
+    int16_t q14[kHeadDim];
 };
 
-struct ExactArgs {
-    StepArgs step;
-    uint32_t exp_lut[33];     // RNE(2^(30 + i/32)), i = 0..32 (cpp:185-195)
+struct KBlock {
+    v4i k[kRows];
+    v2u s[kRows];
+};
+struct VBlock {
+    v4i v[kRows];
 };
 
-// SLICES workgroups share a (sequence, head): each runs the whole token loop
-// (scores, coefficients, Z) but Y for kHeadDim / SLICES channels only, so a
-// small batch spreads over more CUs.  All of them append the new row; they
-// write the same bytes.
-template <bool Q17, int SLICES>
-__global__ __launch_bounds__(256) void exact_kernel(ExactArgs ea) {
-    static_assert(SLICES == 1 || SLICES == 2 || SLICES == 4, "128, 64 or 32 channels per workgroup");
-    // Y roles: threads [0, kCh) run the ordered part (one channel each),
-    // threads [kSeqLanes, 256) compose kCompParts parts of kCh channels,
-    // threads in between (wave 0's upper half when kCh = 32) idle.
-    constexpr int kCh = kHeadDim / SLICES;
-    constexpr int kSeqLanes = kCh < 64 ? 64 : kCh;
-    constexpr int kCompParts = (256 - kSeqLanes) / kCh;
-    constexpr int kGroups = kCh / 32;   // G32 groups of this workgroup's channels
-    constexpr bool kPrefetchY = SLICES == 4;   // the Y pass reads a batch ahead (registers allow it)
-    // The ordered part's share of a chunk, measured: 8/16 with one composed
-    // part (9/16 and 10/16 ran up to 3% slower at batch 16), 2/16 with six
-    // (3/16 ran 7% slower at batch 1; the composed runs round up to whole
-    // batches).
-    constexpr int kSeqShare16 = kCompParts == 1 ? 8 : kCompParts == 3 ? 4 : 2;
-    // The longest composed run (the rest of a chunk after the ordered share,
-    // split into kCompParts runs of whole batches): its short-form terms, and
-    // its prefix sums of fused-multiply-add terms, stay within int32.
-    constexpr int kMaxRun =
-        ((kChunk * (16 - kSeqShare16) / 16 + kCompParts - 1) / kCompParts + kBatch - 1) / kBatch * kBatch;
-    static_assert(kMaxRun * kShortTermBound < (int64_t(1) << 31), "short-form sums of a run fit in 32 bits");
-    static_assert(2 * kMaxRun * kFastTermBound < (int64_t(1) << 31), "a run's prefix-sum range fits in 32 bits");
-    const StepArgs& a = ea.step;
-    const uint32_t row = a.rows[blockIdx.y];
-    const int h = blockIdx.x / SLICES, slice = blockIdx.x % SLICES, b = static_cast<int>(row & 0xffu);
-    const int pos = static_cast<int>(row >> 8);
-    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63;
-    const int c = lane & 7, r = lane >> 3;
-    const int d = threadIdx.x;                  // token of the chunk (coefficients), channel (Y, d < 128)
-    int8_t* page = page_ptr(a.kv, a.slot0 + b, a.layer, h);
-    const int64_t cap = a.kv.seq_cap;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        page, static_cast<short>(0), static_cast<int32_t>(cap * kTokenBytes), kBufferWord3);
+// The page through one buffer resource: per-lane offsets fixed, the token
+// offset in an SGPR.  `past` puts a load past the page's range (zeros, no
+// memory access), for a wave without a (further) block.
+struct Page {
+    __amdgpu_buffer_rsrc_t rsrc;
+    int32_t code_lane;       // lane's byte offset in a code plane
+    int32_t scale_lane;      // lane's scale pair
+    int32_t v_plane, s_plane, end;
+};
 
-    // Per token of the chunk: the score, then (each thread rewrites its own
-    // token after reading it) the coefficient word, zero past n.
-    __shared__ __align__(16) uint32_t s_tok[kChunk];
-    __shared__ int8_t s_vc[kChunk][kHeadDim];            // V codes of the chunk
-    // Per group of this workgroup's channels and token of the chunk: the V
-    // scale (the score pass), then the product p = c 2^(s-17) for ordinary
-    // tokens (the coefficient pass).  The rotated query before the token loop
-    // and the A14 codes after it use the same bytes.
-    __shared__ __align__(16) std::conditional_t<SLICES == 1, ProductsOrQuery<kGroups, kCh>, ProductsAndQuery<kGroups, kCh>>
-        s_u;
-    __shared__ int32_t s_wave_max[kChunk / 64];
-    __shared__ uint32_t s_wave_sum[kChunk / 64];
-    // Per-wave ballots: first and rescaling tokens; those and tokens with a V
-    // shift of 16 or more in this workgroup's groups (the slow form); tokens
-    // with a shift of 17 or more.
-    __shared__ uint64_t s_special[kChunk / 64];
-    __shared__ uint64_t s_slow[kChunk / 64];
-    __shared__ uint64_t s_wide17[kChunk / 64];
-    __shared__ int64_t s_map_sum[kCompParts * kCh];      // the composed maps of the parts after split
-    __shared__ int32_t s_map_lo[kCompParts * kCh];
-    __shared__ int32_t s_map_hi[kCompParts * kCh];
-    __shared__ uint32_t s_lut[33];
-    __shared__ uint32_t s_inv;
-    int32_t* const s_q = s_u.q;
-    int16_t* const s_q14 = s_u.q14;
-    if (threadIdx.x < 33) s_lut[threadIdx.x] = ea.exp_lut[threadIdx.x];
+constexpr int kNontemporal = 2;
 
-    // Wave 0 rotates the query into LDS and appends the new row; the barrier
-    // makes the row visible to the workgroup (its waves share one CU), so the
-    // token loop below reads tokens [0, pos] uniformly from the cache.
-    if (wave == 0) {
-        const size_t row_elem = static_cast<size_t>(b) * kModelDim + h * kHeadDim + 2 * lane;
-        const int2 cs = a.lut[static_cast<size_t>(pos) * kRopePairs + lane];
-        const int2 qi = load_pair<Q17>(a.q, row_elem);
-        const int2 ki = load_pair<Q17>(a.k, row_elem);
-        const int2 vi = load_pair<Q17>(a.v, row_elem);
-        int32_t q0, q1, k0, k1;
-        rope_pair(qi.x, qi.y, cs, q0, q1);
-        rope_pair(ki.x, ki.y, cs, k0, k1);
-        (void)append_row_codes(page, a.kv.seq_cap, pos, lane, k0, k1, vi.x, vi.y);
-        s_q[2 * lane] = q0;
-        s_q[2 * lane + 1] = q1;
-    }
-    __syncthreads();
-    QueryLimbs ql;
-    {
-        int32_t qc[16];
+__device__ __forceinline__ void load_k_row(const Page& pg, int t, int32_t past, v4i& k, v2u& s) {
+    k = __builtin_amdgcn_raw_buffer_load_b128(pg.rsrc, pg.code_lane + past, t * kCodeBytes, kNontemporal);
+    s = __builtin_amdgcn_raw_buffer_load_b64(pg.rsrc, pg.scale_lane + past, pg.s_plane + t * kScaleBytes, kNontemporal);
+}
+__device__ __forceinline__ void load_v_row(const Page& pg, int t, int32_t past, v4i& v) {
+    v = __builtin_amdgcn_raw_buffer_load_b128(pg.rsrc, pg.code_lane + past, pg.v_plane + t * kCodeBytes, kNontemporal);
+}
+__device__ __forceinline__ void load_k(const Page& pg, int t0, bool any, KBlock& kb) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) qc[j] = s_q[16 * c + j];
-        ql = split_query(qc);
-    }
-    if constexpr (SLICES == 1) __syncthreads();   // the score pass below writes the query's bytes (s_u)
-    // Limbs 3 and 4 zero in every lane of the wave: three-limb dot products.
-    // (With four workgroups per head, at batch 1 and 2, the branch measured
-    // 1% slower, so those launches keep five.)
-    const bool q3 = SLICES == 1 &&
-                    __builtin_amdgcn_ballot_w64((ql.w[3][0] | ql.w[3][1] | ql.w[3][2] | ql.w[3][3] | ql.w[4][0] |
-                                                 ql.w[4][1] | ql.w[4][2] | ql.w[4][3]) != 0) == 0;
-
-    const int len = pos + 1;
-    int32_t run_max = INT32_MIN;   // prefix maximum before the chunk (every thread)
-    uint32_t z = 0;                // Z (wave 3, uniform)
-    int32_t y = 0;                 // Y of channel slice * kCh + d (threads d < kCh)
-    // A chunk's loads, 4 waves x 8 token rows per pass: per lane the K codes
-    // and scale pair into registers, and the V codes straight into LDS (lane
-    // l of a wave writes bytes [16 l, 16 l + 16) of its 8 rows, which is
-    // channel chunk c of row r), all passes at once.  Rows past the chunk's
-    // end load its last token (inside the page) and are not used.  The page
-    // is read through one buffer resource: per-lane 32-bit offsets within the
-    // chunk, the chunk's own offset in an SGPR.
-    v4i kq[kPasses];
-    v2u scl[kPasses];
-    auto issue = [&](int tc, bool with_k, bool with_v) {   // flags are compile-time at every call
-        const int nc = min(kChunk, len - tc);
-        const int32_t k_chunk = tc * kCodeBytes, v_chunk = static_cast<int32_t>(cap + tc) * kCodeBytes;
-        const int32_t s_chunk = static_cast<int32_t>(cap * 2 * kCodeBytes) + tc * kScaleBytes;
+    for (int i = 0; i < kRows; ++i) load_k_row(pg, t0 + 8 * i, any ? 0 : pg.end, kb.k[i], kb.s[i]);
+    __builtin_amdgcn_sched_barrier(0);
+}
+__device__ __forceinline__ void load_v(const Page& pg, int t0, bool any, VBlock& vb) {
 #pragma unroll
-        for (int ps = 0; ps < kPasses; ++ps) {
-            const int32_t tr = min(wave * 8 + r + 32 * ps, nc - 1);
-            if (with_k) {
-                scl[ps] = __builtin_amdgcn_raw_buffer_load_b64(rsrc, tr * kScaleBytes + (c >> 1) * 8, s_chunk, 0);
-                kq[ps] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, tr * kCodeBytes + c * 16, k_chunk, 0);
+    for (int i = 0; i < kRows; ++i) load_v_row(pg, t0 + 8 * i, any ? 0 : pg.end, vb.v[i]);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// Scores of a block, lane l getting token l's, and the exponents of its V
+// scales; v_exp is the largest of those the lane holds.
+// Three limbs and shifts up to 25 (every shift a quantized row has) keep each
+// half-group's scaled dot below 2^49, so doubles hold it and the octet's sum
+// exactly; the general form takes five limbs modulo 2^64.
+__device__ __forceinline__ int32_t score_block(const KBlock& kb, const QueryLimbs& ql, bool q3, const Shared& sh,
+                                               uint2* tok, int c, int r, int lane, int32_t& v_exp) {
+    double own_f = 0.0;
+    int64_t own_i = 0;
+    uint32_t general = 0, vs = 0;      // pairs of rows in the general form; largest V scale
+#pragma unroll
+    for (int i = 0; i < kRows; i += 2) {
+        if ((c & 1) == 0) {
+            reinterpret_cast<uint8_t*>(&tok[8 * i + r].y)[c >> 1] = static_cast<uint8_t>(kb.s[i].y >> 23);
+            reinterpret_cast<uint8_t*>(&tok[8 * i + 8 + r].y)[c >> 1] = static_cast<uint8_t>(kb.s[i + 1].y >> 23);
+        }
+        vs = max(vs, max(kb.s[i].y, kb.s[i + 1].y));
+        if (q3 && __builtin_amdgcn_ballot_w64(max(kb.s[i].x, kb.s[i + 1].x) >= (136u << 23)) == 0) {
+            double t[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const double f = static_cast<double>(__uint_as_float(kb.s[i + u].x));   // 2^(shift-17)
+                t[u] = octet_sum_f64(__builtin_floor(limb_dot3(ql, kb.k[i + u]) * f * 128.0));
             }
-            if (with_v)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    rsrc, (__attribute__((address_space(3))) void*)&s_vc[wave * 8 + 32 * ps][0], 16,
-                    tr * kCodeBytes + c * 16, v_chunk, 0, 0);
+            if (c == i) own_f = t[0];
+            if (c == i + 1) own_f = t[1];
+        } else {
+            general |= 3u << i;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                int32_t a3 = 0, a4 = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    a3 = __builtin_amdgcn_sdot4(static_cast<int32_t>(sh.limb_hi[0][4 * c + j]), kb.k[i + u][j], a3, false);
+                    a4 = __builtin_amdgcn_sdot4(static_cast<int32_t>(sh.limb_hi[1][4 * c + j]), kb.k[i + u][j], a4, false);
+                }
+                const int64_t s = static_cast<int64_t>(limb_dot3(ql, kb.k[i + u])) + (static_cast<int64_t>(a3) << 24) +
+                                  (static_cast<int64_t>(a4) << 32);
+                const int64_t t = octet_sum64(scaled_half(s, shift_of(__uint_as_float(kb.s[i + u].x))));
+                if (c == i + u) own_i = t;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    v_exp = static_cast<int32_t>(vs >> 23);
+    const int32_t score = score_of((general >> c) & 1u ? own_i : static_cast<int64_t>(own_f));   // of token 8 c + r
+    return __shfl(score, 8 * (lane & 7) + (lane >> 3));
+}
+
+// A wave's running sums of ordinary terms: per lane 16 channels of chunk c
+// over rows r, r + 8, ... of its blocks.
+struct Sums {
+    uint32_t acc[16];
+    float bound;             // sum of the p of the lane's group
+    uint32_t z;              // coefficients of the lane's own tokens (lane = token)
+    uint32_t rows;           // terms added per channel (each carries kRoundMagicBits)
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] = 0u;
+        bound = 0.0f;
+        z = rows = 0u;
+    }
+};
+
+// Sums stand here, and no load moves across: left alone, the compiler adds a
+// block's terms as one tree, holding all of them, and loads every row first.
+__device__ __forceinline__ void pin(uint32_t* x) {
+    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7]),
+                      "+v"(x[8]), "+v"(x[9]), "+v"(x[10]), "+v"(x[11]), "+v"(x[12]), "+v"(x[13]), "+v"(x[14]),
+                      "+v"(x[15])
+                 :
+                 : "memory");
+}
+
+// The product p of the lane's coefficient and its group's V scale (exact).
+__device__ __forceinline__ float token_product(uint2 w, uint32_t rot) {
+    return __uint_as_float(w.x) * __uint_as_float(__builtin_amdgcn_alignbit(w.y, w.y, rot) & 0x7f800000u);
+}
+
+// Adds the terms of the block's tokens [a, b) (all of them unless MASKED).
+// Two rows at a time, so that one three-operand add takes both terms.
+template <bool MASKED>
+__device__ __forceinline__ void add_terms(const VBlock& vb, const uint2* tok, int r, uint32_t rot, int a, int b,
+                                          Sums& s) {
+    uint2 w[kRows];
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) w[i] = tok[8 * i + r];
+#pragma unroll
+    for (int i = 0; i < kRows; i += 2) {
+        if (!MASKED || (8 * i + 16 > a && 8 * i < b)) {
+            float p[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int t = 8 * (i + u) + r;
+                p[u] = token_product(w[i + u], rot);
+                if (MASKED && (t < a || t >= b)) p[u] = 0.0f;
+                s.bound += p[u];
+            }
+            s.rows += 2;
+            v4i v0 = vb.v[i], v1 = vb.v[i + 1];
+            if (MASKED) asm volatile("" : "+v"(v0), "+v"(v1));   // as in add_wide_terms
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int32_t c0 = static_cast<int8_t>(v0[j >> 2] >> (8 * (j & 3)));
+                const int32_t c1 = static_cast<int8_t>(v1[j >> 2] >> (8 * (j & 3)));
+                s.acc[j] += term_bits(c0, p[0]) + term_bits(c1, p[1]);
+            }
+            pin(s.acc);
+        }
+    }
+}
+
+// The terms of a block with a V shift of 16 or more.  code p is exact in FP32
+// (at most 24 significant bits), so rint rounds it to nearest even; shifts of
+// 24 and more, whose terms may leave the int32 range, make the bound infinite.
+// The empty asm keeps the compiler from sharing the conversions with the other
+// form: hoisted above the choice between them they would hold 128 registers.
+__device__ __forceinline__ void add_wide_terms(VBlock& vb, const uint2* tok, int r, uint32_t rot, int a, int b,
+                                               Sums& s) {
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int t = 8 * i + r;
+        const uint2 w = tok[t];
+        const float p = t >= a && t < b ? token_product(w, rot) : 0.0f;
+        s.bound += p;
+        if ((__builtin_amdgcn_alignbit(w.y, w.y, rot) & 0x7f800000u) >= __float_as_uint(kHugeScale)) s.bound = INFINITY;
+        v4i v = vb.v[i];
+        asm volatile("" : "+v"(v));
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int32_t code = static_cast<int8_t>(v[j >> 2] >> (8 * (j & 3)));
+            s.acc[j] += static_cast<uint32_t>(static_cast<int32_t>(__builtin_rintf(static_cast<float>(code) * p)));
+        }
+        pin(s.acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// Adds a wave's sums to pool entry e and clears them.  The 16 channels' sums
+// over 8 rows reduce by halves: two permlane swaps pair the rows of the upper
+// and lower half-waves and of the odd and even 16-lane rows while the channels
+// spread over them, and a rotation adds the last pair.
+__device__ __forceinline__ void flush(Shared& sh, int e, Sums& s, int lane) {
+    asm volatile("" : "+v"(lane));   // keeps the addresses below out of registers across the loop around the call
+    const uint32_t magic = s.rows * kRoundMagicBits;
+    uint32_t h8[8], h4[4];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const auto x = __builtin_amdgcn_permlane32_swap(s.acc[j] - magic, s.acc[j + 8] - magic, false, false);
+        h8[j] = x[0] + x[1];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const auto x = __builtin_amdgcn_permlane16_swap(h8[j], h8[j + 4], false, false);
+        h4[j] = x[0] + x[1];
+        h4[j] += dpp_u<kDppRowRor8>(h4[j]);
+    }
+    // lane: channels 8 (lane >> 5) + 4 ((lane >> 4) & 1) + 0..3 of chunk c, two of them per bit 3
+    const int c = lane & 7, up = (lane >> 3) & 1;
+    const int ch = 16 * c + 8 * (lane >> 5) + 4 * ((lane >> 4) & 1) + 2 * up;
+    atomicAdd(reinterpret_cast<uint32_t*>(&sh.pool[e][ch]), up ? h4[2] : h4[0]);
+    atomicAdd(reinterpret_cast<uint32_t*>(&sh.pool[e][ch + 1]), up ? h4[3] : h4[1]);
+    const float bound = across_octets_sum(s.bound);
+    if ((lane & 7) == lane && (lane & 1) == 0) atomicAdd(&sh.pool_b[e][lane >> 1], bound);
+    const uint32_t z = wave_scan_add(s.z);
+    if (lane == 63) atomicAdd(&sh.pool_z[e], z);
+    s.clear();
+}
+
+// Where |y| plus the bound of a segment's terms stays below 2^31 no partial
+// sum saturates.  The bound: |code| <= 128, half a unit of rounding per term
+// and the roundings of the float sums.
+__device__ __forceinline__ bool bounded(int32_t y, float b) {
+    return __builtin_fabsf(static_cast<float>(y)) + (b * 128.125f + 8192.0f) < 2147483000.0f;
+}
+
+__device__ __forceinline__ uint32_t exps_shift(uint32_t exps, int g) { return ((exps >> (8 * g)) & 0xffu) - 110u; }
+__device__ __forceinline__ uint32_t token_coef(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_fabsf(__uint_as_float(x)));
+}
+
+// Y of channel d over tokens [t0, t1) of the workgroup's range, in order, from
+// the coefficients in LDS and the V codes in the page.  `first` is the sequence
+// position of token 0 of the range.  Called by whole waves.
+__device__ __forceinline__ int32_t run_in_order(const Page& pg, const Shared& sh, int first, int d, int t0, int t1,
+                                                int32_t y) {
+    constexpr int kAhead = 8;
+    const int g = d >> 5;
+    const uint32_t rot = (9u + 8u * static_cast<uint32_t>(g)) & 31u;
+    int32_t next[kAhead];
+    auto load = [&](int t) {   // tokens past t1: in the page or zero, not used
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+            next[j] = __builtin_amdgcn_raw_buffer_load_b8(pg.rsrc, d, pg.v_plane + (first + t + j) * kCodeBytes, 0);
+    };
+    load(t0);
+    for (int t = t0; t < t1; t += kAhead) {
+        int32_t code[kAhead];
+        uint2 w[kAhead];
+        uint32_t odd = 0, huge = 0;   // a special token or a shift of 16 or more; a shift of 24 or more
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) {
+            code[j] = static_cast<int8_t>(next[j]);
+            w[j] = sh.tok[min(t + j, t1 - 1)];
+            const uint32_t scale = __builtin_amdgcn_alignbit(w[j].y, w[j].y, rot) & 0x7f800000u;
+            odd |= (w[j].x >> 31) | static_cast<uint32_t>(scale >= __float_as_uint(kWideScale));
+            huge |= static_cast<uint32_t>(scale >= __float_as_uint(kHugeScale));
+        }
+        load(t + kAhead);
+        if (__builtin_amdgcn_ballot_w64(odd != 0u) == 0 && t + kAhead <= t1) {
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j)
+                y = __builtin_elementwise_add_sat(
+                    y, static_cast<int32_t>(term_bits(code[j], token_product(w[j], rot)) - kRoundMagicBits));
+        } else if (__builtin_amdgcn_ballot_w64(huge != 0u) == 0 && t + kAhead <= t1) {
+            // Y = sat32(RNE(Y m >> 17) + x): m = 1.0 and x the term for an
+            // ordinary token, m the coefficient and x = v for a rescaling one,
+            // m = 0 and x = v for the first.
+            int32_t x[kAhead];
+            uint32_t m[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                const bool special = (w[j].x >> 31) != 0u;
+                m[j] = !special ? 1u << 17 : first + t + j == 0 ? 0u : token_coef(w[j].x);
+                uint2 wx = w[j];
+                if (special) wx.x = __float_as_uint(131072.0f);
+                x[j] = static_cast<int32_t>(__builtin_rintf(static_cast<float>(code[j]) * token_product(wx, rot)));
+            }
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) y = __builtin_elementwise_add_sat(mulq17_wrap(y, m[j]), x[j]);
+        } else {
+#pragma unroll 1
+            for (int j = 0; j < kAhead && t + j < t1; ++j) {
+                const uint2 wj = sh.tok[t + j];
+                int32_t x = code[0];
+#pragma unroll
+                for (int i = 1; i < kAhead; ++i) x = i == j ? code[i] : x;
+                uint32_t word = token_coef(wj.x);
+                if ((wj.x >> 31) != 0u) word = first + t + j == 0 ? kInit : word | kRescale;
+                y = y_step(y, uniform(word), dequant_raw(x, exps_shift(wj.y, g)));
+            }
+        }
+    }
+    return y;
+}
+
+// Y of channel d over `rows` staged tokens from row `at`.
+__device__ __forceinline__ int32_t run_staged(const Shared& sh, uint32_t at, int rows, int d, int32_t y) {
+    constexpr int kAhead = 8;
+    const int lane = d & 63;
+    const uint32_t mult = lane < rows ? sh.stage_mult[at + static_cast<uint32_t>(lane)] : 1u << 17;
+    const uint64_t special = __builtin_amdgcn_ballot_w64(mult != 1u << 17);
+    int32_t next[kAhead];
+    auto load = [&](int r) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) next[j] = sh.stage[at + static_cast<uint32_t>(min(r + j, rows - 1))][d];
+    };
+    load(0);
+    for (int r = 0; r < rows; r += kAhead) {
+        int32_t term[kAhead];
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) term[j] = r + j < rows ? next[j] : 0;
+        load(r + kAhead);
+        const uint32_t sp = static_cast<uint32_t>(special >> r) & 0xffu;
+        if (sp == 0u) {
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) y = __builtin_elementwise_add_sat(y, term[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) {
+                if ((sp >> j) & 1u)
+                    y = mulq17_wrap(y, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mult), r + j)));
+                y = __builtin_elementwise_add_sat(y, term[j]);
+            }
+        }
+    }
+    return y;
+}
+
+// Z over tokens [t0, t1), in order (one wave, lane = token): between special
+// tokens it advances by differences of prefix sums modulo 2^30.
+__device__ __forceinline__ uint32_t z_in_order(const Shared& sh, int first, int lane, int t0, int t1, uint32_t z) {
+    for (int t = t0; t < t1; t += 64) {
+        const uint32_t x = t + lane < t1 ? sh.tok[t + lane].x : 0u;
+        const uint32_t coef = token_coef(x);
+        uint64_t special = __builtin_amdgcn_ballot_w64((x >> 31) != 0u);
+        const int32_t incl = static_cast<int32_t>(wave_scan_add((x >> 31) != 0u ? 0u : coef));
+        uint32_t done = 0;
+        for (; special != 0u; special &= special - 1ull) {
+            const int i = __builtin_ctzll(special);
+            const uint32_t upto = static_cast<uint32_t>(__builtin_amdgcn_readlane(incl, i));
+            const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(coef), i));
+            z = z_step((z + (upto - done)) & kMask30, first + t + i == 0 ? kInit : c | kRescale);
+            done = upto;
+        }
+        z = (z + (static_cast<uint32_t>(__builtin_amdgcn_readlane(incl, 63)) - done)) & kMask30;
+    }
+    return z;
+}
+
+// Tagged words of the split exchange: the launch's tag above a 32-bit value.
+__device__ __forceinline__ void publish(uint64_t* p, uint32_t tag, uint32_t v) {
+    __hip_atomic_store(p, (static_cast<uint64_t>(tag) << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t fetch(const uint64_t* p) {
+    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool current(uint64_t w, uint32_t tag) { return static_cast<uint32_t>(w >> 32) == tag; }
+
+// Rounds of re-reads (about a microsecond each) a split waits for the maxima
+// of the splits before it.  They are resident in every launch the plan makes
+// on an idle GPU; where other work keeps one off it, the split gives up.
+constexpr uint32_t kPrefixPolls = 256;
+
+// A split's slot: its maximum, then its entries.  Entry e holds the sums
+// A[128], the values V[128] of the special token they follow (none for entry
+// 0), and six words {z, word, bounds of the four groups}; those of entries 0
+// and 1 lie together behind the count, so that one load per split, a word per
+// lane, takes them.
+constexpr uint32_t kSlotFailed = 1u << 31;
+constexpr int kSlotMax = 0, kSlotCount = 1, kSlotMisc = 2, kSlotEntries = kSlotMisc + 6 * kExactEntries;
+static_assert(kExactSlotWords >= kSlotEntries + kExactEntries * 2 * kHeadDim, "slot layout");
+__device__ __forceinline__ uint64_t* slot_misc(uint64_t* slot, int e) { return slot + kSlotMisc + 6 * e; }
+__device__ __forceinline__ uint64_t* slot_sums(uint64_t* slot, int e) { return slot + kSlotEntries + e * 2 * kHeadDim; }
+__device__ __forceinline__ uint64_t* slot_values(uint64_t* slot, int e) { return slot_sums(slot, e) + kHeadDim; }
+
+// Argument-block fields used late, loaded while the first blocks are in flight.
+struct Tail {
+    int32_t* out;
+    uint8_t* act_q;
+    uint8_t* act_scale;
+    uint32_t merge_polls;
+    uint32_t merge_tag_skew;
+};
+
+template <bool Q17, bool SPLIT>
+__global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pages, uint32_t geometry,
+                                                         uint32_t dispatch, const void* q_in, const void* k_in,
+                                                         const void* v_in, const int2* lut, const void* aux,
+                                                         StepArgs a) {
+    constexpr int kIn = Q17 ? kInQ17 : kInF32;
+    __shared__ Shared sh;
+    const uint32_t uniform_pos = dispatch & StepPreload::kRowsListed;
+    auto row_of = [&](int z) {
+        return uniform_pos != StepPreload::kRowsListed ? pack_row(z, uniform_pos) : a.rows[z];
+    };
+    // The upper half of `dispatch`: the split's tokens when SPLIT, else the rows
+    // less one and a 32nd of the workgroups (the argument block and the grid's
+    // size are a scalar round trip to host memory away).
+    const int C = static_cast<int>(dispatch >> 16) * kSplitQuantum;
+    const int heads = static_cast<int>((dispatch >> 16 & 0xffu) + 1u) * kHeads;
+    const int stride = static_cast<int>(dispatch >> 24) * kHeads;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    int lane = threadIdx.x & 63, d = threadIdx.x;
+    int c = lane & 7, r = lane >> 3;
+    const int cap = static_cast<int>(geometry & 0xffffu);
+    const int split = SPLIT ? blockIdx.x : 0;
+
+    // The head in work.  [begin, stop) are its cached tokens of this
+    // workgroup; the new token is the last step.
+    uint32_t row = SPLIT ? row_of(blockIdx.z) : row_of(blockIdx.x / kHeads);
+    int h = SPLIT ? blockIdx.y : blockIdx.x % kHeads;
+    int b = static_cast<int>(row & 0xffu), pos = static_cast<int>(row >> 8);
+    if (SPLIT && split * C > pos) return;
+    const int nsplit = SPLIT ? (pos + C) / C : 1;
+    const bool owner = split == nsplit - 1;       // appends the new row
+    const bool whole = nsplit == 1;
+    const int begin = split * C;
+    Page pg;
+    pg.end = cap * kTokenBytes;
+    pg.v_plane = cap * kCodeBytes;
+    pg.s_plane = cap * 2 * kCodeBytes;
+    pg.code_lane = r * kCodeBytes + c * 16;
+    pg.scale_lane = r * kScaleBytes + (c >> 1) * 8;
+    auto page_of = [&](int seq, int head) {
+        int8_t* const page = const_cast<int8_t*>(layer_pages) +
+                             (static_cast<int64_t>(seq) * (geometry >> 16) * kHeads + head) *
+                                 (static_cast<int64_t>(cap) * kTokenBytes);
+        return __builtin_amdgcn_make_buffer_rsrc(page, static_cast<short>(0), pg.end, kBufferWord3);
+    };
+    pg.rsrc = page_of(b, h);
+
+    // All loads of the prologue, then the first K and V blocks, before any math.
+    int2 cs;
+    InPair<kIn> row_q, row_k{}, row_v{};
+    auto blocks_of = [&](int position) {           // blocks of the range
+        return ((SPLIT ? min(C, position - begin) : position) + kBlock - 1) / kBlock;
+    };
+    auto load_inputs = [&](int seq, int head, int position) {
+        const size_t row_elem = static_cast<size_t>(seq) * kModelDim + head * kHeadDim + 2 * lane;
+        cs = lut[static_cast<size_t>(position) * kRopePairs + lane];
+        row_q = load_in<kIn>(q_in, row_elem, 0);
+        if (wave == kWaves - 1) {
+            row_k = load_in<kIn>(k_in, row_elem, 0);
+            row_v = load_in<kIn>(v_in, row_elem, 0);
         }
     };
-    // With SLICES = 4 (the smallest batches, where each chunk's load latency
-    // is exposed) the next chunk's K codes and scales are loaded while this
-    // chunk's coefficient and Y passes run; its V codes, which go to LDS,
-    // follow at the top of its own iteration (the barrier after the scores
-    // waits for every write into LDS, so they cannot be outstanding there).
-    constexpr bool kPrefetch = SLICES > 1;
-    if constexpr (kPrefetch) issue(0, true, false);
-    for (int t0 = 0; t0 < len; t0 += kChunk) {
-        const int n = min(kChunk, len - t0);
-        issue(t0, !kPrefetch, true);
-        // Scores of tokens [t0, t0+n).  Every lane of an octet ends a pass
-        // with its token's sum; lane c keeps pass c's, so each lane scales,
-        // rounds and saturates one sum per chunk.
-        static_assert(kPasses == 8, "one pass per lane of an octet");
-        int64_t own = 0;
-#pragma unroll
-        for (int ps = 0; ps < kPasses; ++ps) {
-            const int i = wave * 8 + r + 32 * ps;
-            const int4 kw = make_int4(kq[ps].x, kq[ps].y, kq[ps].z, kq[ps].w);
-            // the token's sum of its 8 half-groups (lanes 8r .. 8r+7), exact
-            const uint32_t ksh = shift_of(__uint_as_float(scl[ps].x));
-            const int64_t p = octet_sum64(q3 ? half_dot<3>(ql, kw, ksh) : half_dot<5>(ql, kw, ksh));
-            if (c == ps) own = p;
-            // the V scale of group c / 2, its exponent alone (the stored
-            // scales are powers of two); slots past n take the scale of shift
-            // 0 and are read by the Y pass with a zero coefficient
-            if ((c & 1) == 0 && (c >> 1) / kGroups == slice)
-                s_u.p[(c >> 1) % kGroups][i] =
-                    __uint_as_float(i < n ? scl[ps].y & 0x7f800000u : 110u << 23);
-        }
-        {
-            const int i = wave * 8 + r + 32 * c;   // the token of pass c
-            if (i < n) s_tok[i] = static_cast<uint32_t>(score_of(own));
-        }
-        __builtin_amdgcn_s_waitcnt(0);   // the V codes are in LDS before the barrier
-        if constexpr (kPrefetch)
-            if (t0 + kChunk < len) issue(t0 + kChunk, true, false);
-        __syncthreads();
+    uint64_t* const workspace = static_cast<uint64_t*>(const_cast<void*>(aux));
+    uint64_t* const arrival = workspace + kExactTableWords + (static_cast<size_t>(b) * kHeads + h) * kArrivalStride;
+    load_inputs(b, h, pos);
+    KBlock kb;
+    VBlock vb;
+    load_k(pg, begin + wave * kBlock, wave < blocks_of(pos), kb);
+    load_v(pg, begin + wave * kBlock, wave < blocks_of(pos), vb);
+    const uint64_t arrival_word = SPLIT ? fetch(arrival) : 0u;
+    const uint32_t exp_entry = reinterpret_cast<const uint32_t*>(workspace)[lane];
+    const Tail tail{reinterpret_cast<int32_t*>(a.out), a.act_q, a.act_scale, a.merge_polls, a.merge_tag_skew};
+    __builtin_amdgcn_sched_barrier(0);
 
-        // Coefficient words, one token per thread: the exclusive prefix
-        // maximum (wave scan, then the maxima of the waves before) gives each
-        // token's running maximum.  The same pass lays out what Y and Z read:
-        // the coefficient words, the products p of the coefficient and each
-        // group's V scale (the scale alone for first and rescaling tokens),
-        // the per-wave sums of the coefficients of ordinary tokens, and the
-        // per-wave ballots.
-        const int32_t sv = d < n ? static_cast<int32_t>(s_tok[d]) : INT32_MIN;
-        float sc[kGroups];   // the token's V scales, read with its score
-#pragma unroll
-        for (int gl = 0; gl < kGroups; ++gl) sc[gl] = s_u.p[gl][d];
-        const int32_t incl = wave_scan_max(sv);
-        if (lane == 63) s_wave_max[wave] = incl;
-        int32_t excl = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, incl);
-        __syncthreads();
-        int32_t before = run_max;
-        for (int w = 0; w < wave; ++w) before = max(before, s_wave_max[w]);
-        excl = lane == 0 ? before : max(before, excl);
-        const uint32_t word = d >= n ? 0u : (t0 == 0 && d == 0) ? kInit : coef_word(sv, excl, s_lut);
-        const bool special = (word & (kInit | kRescale)) != 0u;
-        const uint32_t psum = wave_scan_add(special ? 0u : (word & kCoefMask));
-        const uint64_t special_mask = __ballot(special);
-        const float cf = static_cast<float>(word & kCoefMask);
-        bool wide16 = false, wide17 = false;   // a V shift of 16 (scale 2^-1) or more, of 17 (2^0) or more
-#pragma unroll
-        for (int gl = 0; gl < kGroups; ++gl) {
-            wide16 |= sc[gl] >= 0.5f;
-            wide17 |= sc[gl] >= 1.0f;
-            s_u.p[gl][d] = special ? sc[gl] : cf * sc[gl];   // exact: an integer below 2^18 times a power of two
+    for (int turn = 1;; ++turn) {
+    // Derived per turn: what depends on the lane alone would otherwise stand in
+    // registers through the whole loop, hundreds of addresses.
+    asm volatile("" : "+v"(lane), "+v"(d));
+    c = lane & 7;
+    r = lane >> 3;
+    pg.code_lane = r * kCodeBytes + c * 16;
+    pg.scale_lane = r * kScaleBytes + (c >> 1) * 8;
+    const int stop = SPLIT ? min(begin + C, pos) : pos;
+    const int nblk = blocks_of(pos), own_blocks = wave < nblk ? (nblk - wave + kWaves - 1) / kWaves : 0;
+    // The next head: its first blocks are loaded behind this one's last.
+    int next_b = b, next_h = h, next_pos = 0;
+    bool more = false;
+    if constexpr (!SPLIT) {
+        const int slot = static_cast<int>(blockIdx.x);
+        const int index = turn * stride + ((turn & 1) ? stride - 1 - slot : slot);
+        more = index < heads;
+        if (more) {
+            const uint32_t row = row_of(index / kHeads);
+            next_h = index % kHeads;
+            next_b = static_cast<int>(row & 0xffu);
+            next_pos = static_cast<int>(row >> 8);
         }
-        const uint64_t slow_mask = __ballot(special || wide16), wide17_mask = __ballot(wide17);
-        s_tok[d] = word;
-        if (lane == 63) s_wave_sum[wave] = psum;
+    }
+    Page next = pg;
+    next.rsrc = page_of(next_b, next_h);
+    const int32_t next_past = more && wave < blocks_of(next_pos) ? 0 : pg.end;
+    for (int i = d; i < kPool * kHeadDim / 4; i += kThreads)
+        reinterpret_cast<int4*>(&sh.pool[0][0])[i] = make_int4(0, 0, 0, 0);
+    if (d < kPool) {
+        sh.pool_z[d] = 0u;
+        *reinterpret_cast<float4*>(sh.pool_b[d]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    if (d == 0) {
+        sh.specials = 0u;
+        sh.staged = 0u;
+        sh.failed = 0u;
+    }
+
+    // Query limbs: lane l splits channels 2l, 2l+1; each lane gathers limbs
+    // 0-2 of its chunk.  limb k+1 = (what limb k leaves) / 256, which is the
+    // arithmetic shift plus limb k's sign bit.
+    QueryLimbs ql;
+    bool q3;
+    {
+        const int2 qi = in_to_q17<kIn>(row_q);
+        int32_t q[2];
+        rope_pair(qi.x, qi.y, cs, q[0], q[1]);
+        uint32_t half[5] = {0u, 0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            int32_t rest = q[i];
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                half[k] |= (static_cast<uint32_t>(rest) & 0xffu) << (8 * i);
+                rest = (rest >> 8) + ((rest >> 7) & 1);
+            }
+        }
+        q3 = __builtin_amdgcn_ballot_w64((half[3] | half[4]) != 0u) == 0;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            const uint32_t dword = half[k] | (dpp_u<kDppQuadXor1>(half[k]) << 16);   // valid at even lanes
+            if (k < 3) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) ql.w[k][j] = static_cast<int32_t>(__shfl(dword, 8 * c + 2 * j));
+            } else if ((lane & 1) == 0) {
+                sh.limb_hi[k - 3][lane >> 1] = dword;   // every wave writes the same words
+            }
+        }
+        if (wave == kWaves - 1) {
+            // The new row: codes and shifts, its score, and the append.
+            const int2 ki = in_to_q17<kIn>(row_k), vi = in_to_q17<kIn>(row_v);
+            int32_t k0, k1;
+            rope_pair(ki.x, ki.y, cs, k0, k1);
+            const RowCodes rc = row_codes(k0, k1, vi.x, vi.y);
+            int64_t dot = static_cast<int64_t>(q[0]) * static_cast<int8_t>(rc.k0) +
+                          static_cast<int64_t>(q[1]) * static_cast<int8_t>(rc.k1);
+            dot = scaled_half(octet_sum64(dot), rc.sk);
+#pragma unroll
+            for (int s = 8; s < 64; s <<= 1) dot += __shfl_xor(dot, s);
+            reinterpret_cast<uint16_t*>(sh.new_code)[lane] = static_cast<uint16_t>(rc.v0 | (rc.v1 << 8));
+            if ((lane & 15) == 0) reinterpret_cast<uint8_t*>(&sh.new_exps)[lane >> 4] = static_cast<uint8_t>(rc.sv + 110u);
+            if (lane == 0) sh.new_score = score_of(dot);
+            if (owner) store_row(pg.rsrc, cap, pos, lane, rc);
+        }
+    }
+    if (more) load_inputs(next_b, next_h, next_pos);
+
+    // K pass.  Rows past `stop` are read (inside the page, or zero) and their
+    // scores dropped.
+    uint32_t wide_blocks = 0;                      // own blocks with a V shift of 16 or more
+    auto take_scores = [&](int blk, int first, int end) -> bool {
+        uint2* const tok = sh.tok + blk * kBlock;
+        int32_t v_exp;
+        const int32_t score = score_block(kb, ql, q3, sh, tok, c, r, lane, v_exp);
+        tok[lane].x = static_cast<uint32_t>(score);
+        const int32_t mx = wave_scan_max(first + blk * kBlock + lane < end ? score : INT32_MIN);
+        v_exp = wave_scan_max(v_exp);
+        if (lane == 63) {
+            sh.blk_max[blk] = mx;
+            sh.blk_exp[blk] = v_exp;
+        }
+        return __builtin_amdgcn_readlane(v_exp, 63) >= static_cast<int32_t>(__float_as_uint(kWideScale) >> 23);
+    };
+    // (One place loads the blocks, also for a wave without any: with several
+    // the compiler gives them different registers, and copying between those
+    // waits for the loads.)
+    for (int it = 0; it == 0 || it < own_blocks; ++it) {
+        if (own_blocks > 0 && take_scores(wave + it * kWaves, begin, stop)) wide_blocks |= 1u << it;
+        const bool here = it + 1 < own_blocks;
+        load_k(here ? pg : next, here ? begin + (wave + (it + 1) * kWaves) * kBlock : wave * kBlock,
+               here || next_past == 0, kb);
+    }
+    if (turn == 1 && d < 33) sh.lut[d] = exp_entry;
+    asm volatile("" ::"s"(tail.out), "s"(tail.act_q), "s"(tail.act_scale), "s"(tail.merge_polls), "s"(tail.merge_tag_skew));
+    __syncthreads();
+
+    // The running maximum before every block (lane = block).
+    const int32_t bm = lane < nblk ? sh.blk_max[lane] : INT32_MIN;
+    const int32_t incl = wave_scan_max(bm);
+    // Both halves of the word keep their registers until here: a register the
+    // compiler reuses early waits for the load that still fills it.
+    if (SPLIT) asm volatile("" ::"v"(arrival_word));
+    const uint32_t tag = static_cast<uint32_t>(arrival_word >> 32) + 1u;
+    const uint32_t want = tag + tail.merge_tag_skew;
+    uint64_t* const slots =
+        workspace + kExactTableWords + kExactArrivalWords + (exact_first_slot(b) * kHeads + h * exact_row_slots(b)) * static_cast<size_t>(kExactSlotWords);
+    uint64_t* const mine = slots + split * kExactSlotWords;
+    int32_t before_range = INT32_MIN;
+    if (SPLIT && !whole) {
+        if (wave == 0) {
+            if (lane == 63) publish(mine + kSlotMax, tag, static_cast<uint32_t>(incl));
+            int32_t m = INT32_MIN;
+            bool ok = true;
+            if (lane < split) {
+                const uint64_t* p = slots + lane * kExactSlotWords + kSlotMax;
+                uint64_t w = fetch(p);
+                for (uint32_t n = 0; !current(w, want); ++n) {
+                    if (n >= min(kPrefixPolls, tail.merge_polls)) {
+                        ok = false;
+                        break;
+                    }
+                    __builtin_amdgcn_s_sleep(1);
+                    w = fetch(p);
+                }
+                m = static_cast<int32_t>(static_cast<uint32_t>(w));
+            }
+            m = wave_scan_max(m);
+            if (lane == 63) sh.prefix = m;
+            if (!ok) sh.failed = 1u;
+        }
+        __syncthreads();
+        before_range = uniform(sh.prefix);
+    }
+    int32_t before = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, incl);
+    before = lane == 0 ? before_range : max(before, before_range);
+    const uint64_t hot = __builtin_amdgcn_ballot_w64(lane < nblk && (bm > before || (begin == 0 && lane == 0)));
+    // A stretch whose sum could saturate Y as far as its bound tells is run
+    // token by token, so where coefficients stay near 1.0 over many tokens of
+    // large V the stretches are cut, at every 8th block or at every block.
+    // Lane = block: 64 terms of at most 128 2^shift times the largest
+    // coefficient.
+    uint64_t cuts = 0;
+    {
+        const float coef = fast_exp2((static_cast<float>(min(bm, before)) - static_cast<float>(before)) *
+                                     (1.4426950408889634f * 0x1p-17f));
+        const float most = lane < nblk ? ldexpf(coef, sh.blk_exp[lane] - 110 + 13) : 0.0f;
+        const float eight = octet_sum(most);
+        if (uniform(__float_as_int(across_octets_sum(eight))) >= __float_as_int(0x1p30f))
+            cuts = uniform(__float_as_int(across_octets_max(eight))) >= __float_as_int(0x1p30f) ? ~1ull : 0x0101010101010100ull;
+        if (nblk < 64) cuts &= (1ull << nblk) - 1ull;
+    }
+    const uint64_t bounds = hot | cuts;            // where stretches end
+    const int nbound = __builtin_popcountll(bounds);
+    int32_t top = max(before_range, __builtin_amdgcn_readlane(incl, 63));   // running maximum before the new token
+    // Whether the fold can start at the range's first token: a hot block is
+    // then run in order from its V codes (staged in LDS for the first few);
+    // other splits sum the pieces between its special tokens.
+    const bool folds = !SPLIT || split == 0;
+    static_assert(kMaxBlocks + 1 + kSpecials <= kPool, "an accumulator per stretch and per special token");
+
+    // V pass.  First the coefficient words of a block's tokens (lane = token);
+    // `start` is the running maximum before the block.
+    auto take_words = [&](int blk, int first, int end, int32_t start, bool is_hot) -> uint32_t {
+        uint2* const tok = sh.tok + blk * kBlock;
+        const bool valid = first + blk * kBlock + lane < end;
+        const int32_t score = static_cast<int32_t>(tok[lane].x);
+        int32_t pm = start;                        // running maximum before the lane's token
+        if (is_hot) {
+            pm = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, wave_scan_max(valid ? score : INT32_MIN));
+            pm = lane == 0 ? start : max(pm, start);
+        }
+        const bool init = first + blk + lane == 0;
+        const uint32_t word = !valid ? 0u : init ? kInit : coef_word(score, pm, sh.lut);
+        tok[lane].x = __float_as_uint(static_cast<float>(word & kCoefMask)) |
+                      ((word & (kInit | kRescale)) != 0u ? 0x80000000u : 0u);
+        wave_lds_sync();
+        return word;
+    };
+    const uint32_t rot = (9u + 8u * static_cast<uint32_t>(c >> 1)) & 31u;   // exponent byte c / 2 to bits 23..30
+    Sums s;
+    s.clear();
+    int stretch = 0;                               // hot blocks before the sums in hand
+    bool dirty = false;
+    for (int it = 0; it == 0 || it < own_blocks; ++it) {
+    if (own_blocks > 0) {
+        // The stretch the block's first tokens belong to: after the bound at
+        // its start, if that is a cut, before it if the block is hot.
+        const int blk = wave + it * kWaves;
+        const bool is_hot = (hot >> blk) & 1ull, is_cut = !is_hot && ((cuts >> blk) & 1ull) != 0u;
+        int k = __builtin_popcountll(bounds & ((1ull << blk) - 1ull));
+        if (is_cut) {
+            if (folds && lane == 0) sh.hot[k] = make_uint4(static_cast<uint32_t>(blk * kBlock) * 0x10001u, 0u, 0u, 0u);
+            if (!folds && lane == 0) sh.hot_count[k] = 0u;
+            ++k;
+        }
+        if (k != stretch && dirty) {
+            flush(sh, stretch, s, lane);
+            dirty = false;
+        }
+        stretch = k;
+        const bool wide = (wide_blocks >> it) & 1u;
+        const uint2* const tok = sh.tok + blk * kBlock;
+        const uint32_t word = take_words(blk, begin, stop, __builtin_amdgcn_readlane(before, blk), is_hot);
+        const uint32_t coef = word & kCoefMask;
+        if (!is_hot) {
+            s.z += coef;
+            if (!wide) add_terms<false>(vb, tok, r, rot, 0, kBlock, s);
+            else add_wide_terms(vb, tok, r, rot, 0, kBlock, s);
+            dirty = true;
+        } else if (folds) {
+            // From the first to the last special token the block is run in
+            // order later; the tokens before join the stretch that ends here,
+            // those after the next one.
+            const uint64_t m = __builtin_amdgcn_ballot_w64((word & (kInit | kRescale)) != 0u);
+            const int t_first = __builtin_ctzll(m), t_last = 63 - __builtin_clzll(m);
+            const int rows = t_last - t_first + 1;
+            uint32_t at = kStageRows;
+            const uint2 own = tok[lane];
+            const bool special = (own.x >> 31) != 0u;
+            const uint32_t widest = max(max(own.y & 0xffu, (own.y >> 8) & 0xffu), max((own.y >> 16) & 0xffu, own.y >> 24));
+            const bool huge = __builtin_amdgcn_ballot_w64(widest >= __float_as_uint(kHugeScale) >> 23) != 0;
+            if (!huge && lane == 0) at = atomicAdd(&sh.staged, static_cast<uint32_t>(rows));
+            at = uniform(at);
+            if (lane == t_first)
+                sh.hot[k] = make_uint4(static_cast<uint32_t>(blk * kBlock + t_first) |
+                                           static_cast<uint32_t>(blk * kBlock + t_last + 1) << 16,
+                                       at, (word & kInit) ? 0u : coef, 0u);
+            if (at + static_cast<uint32_t>(rows) <= static_cast<uint32_t>(kStageRows)) {
+                if (lane >= t_first && lane <= t_last)
+                    sh.stage_mult[at + static_cast<uint32_t>(lane - t_first)] =
+                        !special ? 1u << 17 : (word & kInit) ? 0u : coef;
+#pragma unroll
+                for (int i = 0; i < kRows; ++i) {
+                    const int t = 8 * i + r;
+                    uint2 w = tok[t];
+                    if ((w.x >> 31) != 0u) w.x = __float_as_uint(131072.0f);   // v itself: 2^17 scale = 2^shift
+                    const float p = token_product(w, rot);
+                    v4i v = vb.v[i];
+                    asm volatile("" : "+v"(v));   // as in add_wide_terms
+                    if (t >= t_first && t <= t_last) {
+                        v4i* const out = reinterpret_cast<v4i*>(&sh.stage[at + static_cast<uint32_t>(t - t_first)][16 * c]);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            v4i x;
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                x[j] = static_cast<int32_t>(__builtin_rintf(
+                                    static_cast<float>(static_cast<int8_t>(v[q] >> (8 * j))) * p));
+                            out[q] = x;
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            for (int part = 0; part < 2; ++part) {
+                const int from = part == 0 ? 0 : t_last + 1, to = part == 0 ? t_first : kBlock;
+                if (to > from) {
+                    s.z += lane >= from && lane < to ? coef : 0u;
+                    if (wide) add_wide_terms(vb, tok, r, rot, from, to, s);
+                    else add_terms<true>(vb, tok, r, rot, from, to, s);
+                    dirty = true;
+                }
+                if (part == 0 && dirty) {
+                    flush(sh, k, s, lane);
+                    dirty = false;
+                }
+            }
+            stretch = k + 1;
+        } else if constexpr (SPLIT) {
+            // The block's special tokens, and the pieces between them: the
+            // first piece joins the stretch.
+            const bool special = (word & (kInit | kRescale)) != 0u;
+            uint64_t m = __builtin_amdgcn_ballot_w64(special);
+            const int count = __builtin_popcountll(m);
+            uint32_t first = 0;
+            if (lane == 0) first = atomicAdd(&sh.specials, static_cast<uint32_t>(count));
+            first = uniform(first);
+            if (first + count > static_cast<uint32_t>(kSpecials) || wide) {
+                if (lane == 0) sh.failed = 1u;
+            } else {
+                if (lane == 0) {
+                    sh.hot_first[k] = first;
+                    sh.hot_count[k] = static_cast<uint32_t>(count);
+                }
+                int e = k;
+                for (int from = 0;;) {
+                    const int t = m != 0u ? __builtin_ctzll(m) : kBlock;
+                    if (t > from) {
+                        s.z += lane >= from && lane < t ? coef : 0u;
+                        add_terms<true>(vb, tok, r, rot, from, t, s);
+                        dirty = true;
+                    }
+                    if (dirty) flush(sh, e, s, lane);
+                    dirty = false;
+                    if (m == 0u) break;
+                    const uint32_t idx = first + static_cast<uint32_t>(count - __builtin_popcountll(m));
+#pragma unroll
+                    for (int i = 0; i < kRows; ++i)
+                        if (i == t >> 3 && r == (t & 7)) *reinterpret_cast<v4i*>(&sh.code[idx][16 * c]) = vb.v[i];
+                    if (lane == t) {
+                        sh.sp_word[idx] = word;
+                        sh.sp_exps[idx] = tok[lane].y;
+                    }
+                    e = kPool - 1 - static_cast<int>(idx);
+                    from = t + 1;
+                    m &= m - 1ull;
+                }
+            }
+            if (dirty) flush(sh, k, s, lane);
+            dirty = false;
+            stretch = k + 1;
+        }
+    }
+        const bool here = it + 1 < own_blocks;
+        load_v(here ? pg : next, here ? begin + (wave + (it + 1) * kWaves) * kBlock : wave * kBlock,
+               here || next_past == 0, vb);
+    }
+    if (dirty) flush(sh, stretch, s, lane);
+    __syncthreads();
+    const bool usable = uniform(sh.failed) == 0u;
+
+    // The fold: the stretches' sums and the hot blocks in token order, one
+    // thread per channel for Y, one wave for Z.
+    const int g = (d >> 5) & 3;
+    int32_t y = 0;
+    uint32_t z = 0;
+    const int32_t new_v = dequant_raw(sh.new_code[d & (kHeadDim - 1)], exps_shift(sh.new_exps, g));
+    if (wave < 2 && folds) {
+        // Stretch k, then hot block k's span, often one token; what block k + 1
+        // needs is read ahead.
+        const uint4 table = sh.hot[lane];
+        auto column = [&](uint32_t x, int k) {
+            return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), k));
+        };
+        const int n = usable ? nbound : 0;
+        int32_t sum = sh.pool[0][d], first = sh.stage[min(column(table.y, 0), kStageRows - 1u)][d];
+        float bound = sh.pool_b[0][g];
+        int from = 0;
+        for (int k = 0;; ++k) {
+            const int32_t sum_k = sum, first_k = first;
+            const float bound_k = bound;
+            const int kn = min(k + 1, n);
+            sum = sh.pool[kn][d];
+            bound = sh.pool_b[kn][g];
+            first = sh.stage[min(column(table.y, kn & 63), kStageRows - 1u)][d];
+            const uint32_t span = column(table.x, k & 63), at = column(table.y, k & 63);
+            const int span0 = k < n ? static_cast<int>(span & 0xffffu) : stop - begin;
+            if (usable && __builtin_amdgcn_ballot_w64(!bounded(y, bound_k)) == 0) y += sum_k;
+            else y = run_in_order(pg, sh, begin, d, from, span0, y);
+            if (k == n) break;
+            from = static_cast<int>(span >> 16);
+            const int rows = from - span0;         // none at a cut
+            if (rows == 0) continue;
+            if (at + static_cast<uint32_t>(rows) <= static_cast<uint32_t>(kStageRows)) {
+                y = __builtin_elementwise_add_sat(mulq17_wrap(y, column(table.z, k)), first_k);
+                if (rows > 1) y = run_staged(sh, at + 1u, rows - 1, d, y);
+            } else {
+                y = run_in_order(pg, sh, begin, d, span0, from, y);
+            }
+        }
+    } else if (wave == 2) {
+        const uint32_t word = pos == 0 ? kInit : coef_word(sh.new_score, top, sh.lut);
+        if (folds) {
+            const uint4 table = sh.hot[lane];
+            const uint32_t zs = sh.pool_z[lane], z_last = sh.pool_z[64];
+            if (!usable) z = z_in_order(sh, begin, lane, 0, stop - begin, z);
+            for (int k = 0; usable; ++k) {
+                z = (z + (k < 64 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(zs), k)) : z_last)) &
+                    kMask30;
+                if (k == nbound) break;
+                const uint32_t span = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(table.x), k));
+                const uint32_t mult = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(table.z), k));
+                const int span0 = static_cast<int>(span & 0xffffu), span1 = static_cast<int>(span >> 16);
+                if (span0 == span1) continue;
+                z = z_step(z, begin + span0 == 0 ? kInit : mult | kRescale);
+                if (span0 + 1 < span1) z = z_in_order(sh, begin, lane, span0 + 1, span1, z);
+            }
+            if (whole) z = z_step(z, word);
+        }
         if (lane == 0) {
-            s_special[wave] = special_mask;
-            s_slow[wave] = slow_mask;
-            s_wide17[wave] = wide17_mask;
+            sh.z = z;
+            sh.new_word = word;
         }
-#pragma unroll
-        for (int w = 0; w < kChunk / 64; ++w) run_max = max(run_max, s_wave_max[w]);
-        __syncthreads();
+    }
+    __syncthreads();
+    z = sh.z;
+    const uint32_t new_word = uniform(sh.new_word);
+    if (whole && wave < 2) y = y_step(y, new_word, new_v);
 
-        // Y in parts at once.  Threads [0, kCh) (one channel each) run
-        // tokens [0, split) in order; the composing threads split [split, n)
-        // into kCompParts runs of q tokens and compose each run into one map
-        // Y -> clamp(Y + A, L, H) (every ordinary token is Y -> sat32(Y + t),
-        // and such maps compose: A adds t, L and H take sat32(. + t)), which
-        // the ordered threads apply in order after the barrier.  A batch or
-        // run with a first or rescaling token, or a shift of 16 or more,
-        // takes the slow form (the ballots say which).  split is
-        // about kSeqShare16/16 of n, past the chunk's last first or rescaling
-        // token, and a multiple of kBatch, and so is q.  Slots past n have a
-        // zero coefficient, so a zero term.
-        const int split0 = min(n, ((n * kSeqShare16) / 16 + kBatch - 1) & ~(kBatch - 1));
-        int last_special = -1;
-#pragma unroll
-        for (int w = 0; w < kChunk / 64; ++w) {
-            const int lo = split0 - 64 * w;
-            if (lo < 64) {
-                uint64_t m = uniform64(s_special[w]);
-                if (lo > 0) m &= ~0ull << lo;
-                if (m != 0u) last_special = 64 * w + 63 - __builtin_clzll(m);
+    if (SPLIT && !whole) {
+        // Publish the range's entries; a split that cannot only says so.  Its own
+        // sums of entries 0 and 1 stay at hand, in case it is the one that folds.
+        uint32_t own_a0 = 0, own_a1 = 0, own_v1 = 0;
+        if (wave < 2) {
+            int entries = 1;
+            auto put = [&](int e, uint32_t av, uint32_t zv, float bv) {
+                publish(slot_sums(mine, e) + d, tag, av);
+                if (d == 0) publish(slot_misc(mine, e), tag, zv);
+                if ((d & 31) == 0) publish(slot_misc(mine, e) + 2 + g, tag, __float_as_uint(bv));
+                if (e == 0) own_a0 = av;
+                if (e == 1) own_a1 = av;
+                if (e < 2 && d == 0) sh.misc[1 + 6 * e] = zv;
+                if (e < 2 && (d & 31) == 0) sh.misc[3 + 6 * e + g] = __float_as_uint(bv);
+            };
+            auto put_special = [&](int e, uint32_t word, int32_t v) {
+                publish(slot_values(mine, e) + d, tag, static_cast<uint32_t>(v));
+                if (d == 0) publish(slot_misc(mine, e) + 1, tag, word);
+                if (e == 1) own_v1 = static_cast<uint32_t>(v);
+                if (e < 2 && d == 0) sh.misc[2 + 6 * e] = word;
+            };
+            if (folds) {
+                put(0, static_cast<uint32_t>(y), z, 0.0f);
+            } else if (usable && static_cast<int>(uniform(sh.specials)) + __builtin_popcountll(cuts & ~hot) + 1 +
+                                        (owner ? 1 : 0) <= kExactEntries) {
+                put(0, static_cast<uint32_t>(sh.pool[0][d]), sh.pool_z[0], sh.pool_b[0][g]);
+                for (int k = 0; k < nbound; ++k) {
+                    const uint32_t first = uniform(sh.hot_first[k]), count = uniform(sh.hot_count[k]);
+                    if (count == 0u) {             // a cut: an ordinary token that adds nothing
+                        put_special(entries, 0u, 0);
+                        put(entries, static_cast<uint32_t>(sh.pool[k + 1][d]), sh.pool_z[k + 1], sh.pool_b[k + 1][g]);
+                        ++entries;
+                    }
+                    for (uint32_t i = 0; i < count; ++i) {
+                        const int idx = static_cast<int>(first + i), e = kPool - 1 - idx;
+                        uint32_t av = static_cast<uint32_t>(sh.pool[e][d]), zv = sh.pool_z[e];
+                        float bv = sh.pool_b[e][g];
+                        if (i + 1 == count) {
+                            av += static_cast<uint32_t>(sh.pool[k + 1][d]);
+                            zv += sh.pool_z[k + 1];
+                            bv += sh.pool_b[k + 1][g];
+                        }
+                        put_special(entries, sh.sp_word[idx],
+                                    dequant_raw(sh.code[idx][d], exps_shift(sh.sp_exps[idx], g)));
+                        put(entries, av, zv, bv);
+                        ++entries;
+                    }
+                }
+                if (owner) {
+                    put_special(entries, new_word, new_v);
+                    put(entries, 0u, 0u, 0.0f);
+                    ++entries;
+                }
+            } else {
+                entries = static_cast<int>(kSlotFailed);
+            }
+            if (d == 0) {
+                publish(mine + kSlotCount, tag, static_cast<uint32_t>(entries));
+                sh.misc[0] = static_cast<uint32_t>(entries);
             }
         }
-        const int split = last_special < 0 ? split0 : (last_special + kBatch) & ~(kBatch - 1);
-        const int rest = n - split;
-        const int q = rest > 0 ? ((rest + kCompParts - 1) / kCompParts + kBatch - 1) & ~(kBatch - 1) : 0;
-        const int cp = d < kSeqLanes ? 0 : (d - kSeqLanes) / kCh;   // composed part of a composing thread
-        const int cl = d < kSeqLanes ? d % kCh : (d - kSeqLanes) % kCh;
-        const int ch = slice * kCh + cl;
-        const float* s_p_g = s_u.p[cl >> 5];   // this channel's group
-        if (d < kCh) {
-            // With four workgroups per head a CU holds one of them, so the
-            // ordered part's LDS latency is exposed: the next batch's reads go
-            // out while this one's terms are formed.
-            FastBatch next;
-            if constexpr (kPrefetchY)
-                if (split > 0) next = load_fast(s_p_g, s_vc, 0, ch);
-            for (int span = 0; span < split; span += 64) {
-                const uint64_t spans = uniform64(s_special[span >> 6]);
-                const uint64_t slows = uniform64(s_slow[span >> 6]);
-                const uint64_t wides = uniform64(s_wide17[span >> 6]);
-                const int end = min(span + 64, split);
-                for (int i0 = span; i0 < end; i0 += kBatch) {
-                    const int at = i0 - span;
-                    FastBatch cur;
-                    if constexpr (kPrefetchY) {
-                        cur = next;
-                        if (i0 + kBatch < split) next = load_fast(s_p_g, s_vc, i0 + kBatch, ch);
-                    }
-                    if (((slows >> at) & kBatchMask) == 0u) {
-                        // No first or rescaling token and every shift at most
-                        // 15: fused-multiply-add terms.  Where no Y of the
-                        // wave lies within kBatch 2^22 of either end of the
-                        // int32 range no partial sum saturates, and the batch
-                        // adds its terms at once (modulo 2^32, then exact).
-                        if constexpr (!kPrefetchY) cur = load_fast(s_p_g, s_vc, i0, ch);
-                        uint32_t tb[kBatch];
-                        fast_term_bits(cur, tb);
-                        const bool safe = static_cast<uint32_t>(y) + (0x80000000u - kSatMargin) <= ~(2u * kSatMargin);
-                        if (__builtin_amdgcn_ballot_w64(!safe) == 0u) {
-                            uint32_t acc = static_cast<uint32_t>(y) - kBatch * kRoundMagicBits;
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j) acc += tb[j];
-                            y = static_cast<int32_t>(acc);
-                        } else {
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j)
-                                y = __builtin_elementwise_add_sat(y, static_cast<int32_t>(tb[j] - kRoundMagicBits));
-                        }
-                    } else {
-                        int32_t code[kBatch], term[kBatch];
-                        float pv[kBatch];
-                        slow_terms(s_tok, s_p_g, s_vc, i0, ch, ((wides >> at) & kBatchMask) != 0u, code, pv, term);
-                        if (((spans >> at) & kBatchMask) == 0u) {
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j) y = __builtin_elementwise_add_sat(y, term[j]);
-                        } else {
-                            // A first or rescaling token's p is its V scale.
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j) {
-                                const uint32_t w = static_cast<uint32_t>(
-                                    __builtin_amdgcn_readfirstlane(static_cast<int>(s_tok[i0 + j])));
-                                y = value_step(y, w, code[j], shift_of(pv[j]), term[j]);
-                            }
-                        }
-                    }
-                }
-            }
-        } else if (d >= kSeqLanes) {
-            if (wave == 3) {
-                // Z: ordinary tokens add their coefficients modulo 2^30, so
-                // between two first or rescaling tokens Z advances by a
-                // difference of prefix sums, and only those tokens step in
-                // order.  The prefix sums of a 64-token span that holds such
-                // a token come from a wave scan of its coefficient words.
-                uint32_t done = 0u, offset = 0u;   // prefix sum already added; sum of the spans before
-#pragma unroll
-                for (int w = 0; w < kChunk / 64; ++w) {
-                    uint64_t m = uniform64(s_special[w]);
-                    if (m != 0u) {
-                        const uint32_t wd = s_tok[64 * w + lane];
-                        const uint32_t incl = wave_scan_add((wd & (kInit | kRescale)) != 0u ? 0u : (wd & kCoefMask));
-                        while (m != 0u) {
-                            const int i = __builtin_ctzll(m);
-                            // the sum of the ordinary tokens before i (i itself counts zero)
-                            const uint32_t upto =
-                                offset + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), i));
-                            z = (z + (upto - done)) & kMask30;
-                            done = upto;
-                            z = z_step(z, static_cast<uint32_t>(
-                                              __builtin_amdgcn_readfirstlane(static_cast<int>(s_tok[64 * w + i]))));
-                            m &= m - 1u;
-                        }
-                    }
-                    offset += s_wave_sum[w];
-                }
-                z = (z + (offset - done)) & kMask30;
-            }
-            // A composing thread's run [begin, end) holds no first or
-            // rescaling token.  With kCh = 32 a wave holds two parts, so what
-            // depends on the run is read per lane.
-            const int begin = split + cp * q, end = min(n, begin + q);
-            if (begin < n) {
-                // Slow-form tokens in [split, n) (wave-uniform), then, with
-                // two parts per wave, in this lane's run.
-                bool slow_run = false;
-#pragma unroll
-                for (int w = 0; w < kChunk / 64; ++w) {
-                    const int lo_t = max(split - 64 * w, 0), hi_t = min(n - 64 * w, 64);
-                    if (lo_t < hi_t)
-                        slow_run |= (uniform64(s_slow[w]) & (~0ull >> (64 - (hi_t - lo_t))) << lo_t) != 0u;
-                }
-                if (kCompParts > 1 && slow_run) {
-                    slow_run = false;
-#pragma unroll
-                    for (int w = 0; w < kChunk / 64; ++w) {
-                        const int lo_t = max(begin - 64 * w, 0), hi_t = min(end - 64 * w, 64);
-                        if (lo_t < hi_t)
-                            slow_run |= (s_slow[w] & (~0ull >> (64 - (hi_t - lo_t))) << lo_t) != 0u;
-                    }
-                }
-                if (!slow_run) {
-                    // Fused-multiply-add terms.  With prefix sums P_k (P_0 =
-                    // 0) the map is A = P_n, L = INT32_MIN + P_n - min P_k,
-                    // H = INT32_MAX + P_n - max P_k: the sat32 recursion of L
-                    // and H in closed form, exact while neither reaches the
-                    // far end of the int32 range (|P_k| < 2^30, see kMaxRun).
-                    int32_t pk = 0, pmin = 0, pmax = 0;
-                    FastBatch next;
-                    if constexpr (kPrefetchY) next = load_fast(s_p_g, s_vc, begin, ch);
-                    for (int i0 = begin; i0 < end; i0 += kBatch) {
-                        FastBatch cur;
-                        if constexpr (kPrefetchY) {
-                            cur = next;
-                            if (i0 + kBatch < end) next = load_fast(s_p_g, s_vc, i0 + kBatch, ch);
-                        } else {
-                            cur = load_fast(s_p_g, s_vc, i0, ch);
-                        }
-                        uint32_t tb[kBatch];
-                        fast_term_bits(cur, tb);
-#pragma unroll
-                        for (int j = 0; j < kBatch; j += 2) {
-                            const int32_t p1 = pk + static_cast<int32_t>(tb[j] - kRoundMagicBits);
-                            const int32_t p2 = p1 + static_cast<int32_t>(tb[j + 1] - kRoundMagicBits);
-                            pmin = min(pmin, min(p1, p2));
-                            pmax = max(pmax, max(p1, p2));
-                            pk = p2;
-                        }
-                    }
-                    s_map_sum[cp * kCh + cl] = pk;
-                    s_map_lo[cp * kCh + cl] = INT32_MIN + (pk - pmin);
-                    s_map_hi[cp * kCh + cl] = INT32_MAX + (pk - pmax);
-                } else {
-                    int64_t sum = 0;
-                    int32_t sum_short = 0;   // the short-form batches' terms (see kMaxRun)
-                    int32_t lo = INT32_MIN, hi = INT32_MAX;
-                    for (int i0 = begin; i0 < end; i0 += kBatch) {
-                        int32_t code[kBatch], term[kBatch];
-                        float pv[kBatch];
-                        const bool wide = ((s_wide17[i0 >> 6] >> (i0 & 63)) & kBatchMask) != 0u;
-                        if (slow_terms(s_tok, s_p_g, s_vc, i0, ch, wide, code, pv, term)) {
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j) {
-                                sum_short += term[j];
-                                lo = __builtin_elementwise_add_sat(lo, term[j]);
-                                hi = __builtin_elementwise_add_sat(hi, term[j]);
-                            }
-                        } else {
-#pragma unroll
-                            for (int j = 0; j < kBatch; ++j) {
-                                sum += term[j];
-                                lo = __builtin_elementwise_add_sat(lo, term[j]);
-                                hi = __builtin_elementwise_add_sat(hi, term[j]);
-                            }
-                        }
-                    }
-                    sum += sum_short;
-                    s_map_sum[cp * kCh + cl] = sum;
-                    s_map_lo[cp * kCh + cl] = lo;
-                    s_map_hi[cp * kCh + cl] = hi;
-                }
-            }
+        // The count goes out from a wave that publishes nothing.
+        constexpr unsigned kCountThread = kHeadDim;
+        if (threadIdx.x == kCountThread) {
+            const uint64_t n = __hip_atomic_fetch_add(arrival, uint64_t(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            sh.last = static_cast<uint32_t>(n) == static_cast<uint32_t>(nsplit - 1);
+            sh.redo = 0u;
         }
         __syncthreads();
-        if (d < kCh) {
+        if (!uniform(sh.last)) return;
+
+        // The last split of the head to arrive folds the entries of all of
+        // them.  Every split has counted, so its words land by themselves.
+        // Entries 0 and 1 of every split come in one round of loads.
+        if (wave < 2) {
+            bool ok = true;
+            uint32_t budget = tail.merge_polls;
+            constexpr int kMisc = 13;              // the count and the words of entries 0 and 1
+            uint64_t mw[kExactMaxSplits], a0[kExactMaxSplits], a1[kExactMaxSplits], v1[kExactMaxSplits];
+            for (;;) {
 #pragma unroll
-            for (int p = 0; p < kCompParts; ++p) {
-                if (split + p * q >= n) break;
-                const int k = p * kCh + cl;
-                y = static_cast<int32_t>(min(max(static_cast<int64_t>(y) + s_map_sum[k], static_cast<int64_t>(s_map_lo[k])),
-                                             static_cast<int64_t>(s_map_hi[k])));
+                for (int j = 0; j < kExactMaxSplits; ++j) {
+                    const uint64_t own_tag = static_cast<uint64_t>(want) << 32;
+                    mw[j] = own_tag | sh.misc[min(lane, kMisc - 1)];
+                    a0[j] = own_tag | own_a0;
+                    a1[j] = own_tag | own_a1;
+                    v1[j] = own_tag | own_v1;
+                    if (j < nsplit && j != split) {
+                        uint64_t* const p = slots + j * kExactSlotWords;
+                        mw[j] = fetch(p + kSlotCount + min(lane, kMisc - 1));
+                        a0[j] = fetch(slot_sums(p, 0) + d);
+                        a1[j] = fetch(slot_sums(p, 1) + d);
+                        v1[j] = fetch(slot_values(p, 1) + d);
+                    }
+                }
+                bool stale = false;
+#pragma unroll
+                for (int j = 0; j < kExactMaxSplits; ++j) {
+                    if (j < nsplit) {
+                        const uint64_t count = __builtin_amdgcn_readlane(static_cast<int>(mw[j] >> 32), 0) ==
+                                                       static_cast<int>(want)
+                                                   ? uniform(static_cast<uint32_t>(mw[j]))
+                                                   : 0u;
+                        // of a failed split nothing but the count is read
+                        const bool failed = (count & kSlotFailed) != 0u, more = !failed && count > 1u;
+                        stale |= count == 0u || (!failed && !current(a0[j], want)) ||
+                                 (more && (!current(a1[j], want) || !current(v1[j], want))) ||
+                                 (!failed && lane >= 1 && lane < (more ? kMisc : 7) && lane != 2 &&
+                                  !current(mw[j], want));
+                    }
+                }
+                if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
+                if (budget-- == 0u) {
+                    ok = false;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            y = 0;
+            z = 0u;
+#pragma unroll
+            for (int j = 0; j < kExactMaxSplits; ++j) {
+                if (j < nsplit && ok) {
+                    auto misc = [&](int i) -> uint32_t {
+                        return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mw[j]), i));
+                    };
+                    const uint32_t n = misc(0);
+                    auto add = [&](uint32_t sum, uint32_t coefs, uint32_t bound_lo, uint32_t bound_hi) {
+                        const float bv = __uint_as_float((d & 32) ? bound_hi : bound_lo);
+                        ok = ok && __builtin_amdgcn_ballot_w64(!bounded(y, bv)) == 0;
+                        y = static_cast<int32_t>(static_cast<uint32_t>(y) + sum);
+                        z = (z + coefs) & kMask30;
+                    };
+                    if (n & kSlotFailed) {
+                        ok = false;
+                    } else {
+                        add(static_cast<uint32_t>(a0[j]), misc(1), wave ? misc(5) : misc(3), wave ? misc(6) : misc(4));
+                        if (n > 1) {
+                            y = y_step(y, misc(8), static_cast<int32_t>(static_cast<uint32_t>(v1[j])));
+                            z = z_step(z, misc(8));
+                            add(static_cast<uint32_t>(a1[j]), misc(7), wave ? misc(11) : misc(9),
+                                wave ? misc(12) : misc(10));
+                        }
+                        for (uint32_t e = 2; ok && e < n; ++e) {
+                            uint64_t* const p = slots + j * kExactSlotWords;
+                            uint64_t m, sum, v;
+                            for (;;) {
+                                m = fetch(slot_misc(p, static_cast<int>(e)) + min(lane, 5));
+                                sum = fetch(slot_sums(p, static_cast<int>(e)) + d);
+                                v = fetch(slot_values(p, static_cast<int>(e)) + d);
+                                const bool stale = !current(m, want) || !current(sum, want) || !current(v, want);
+                                if (__builtin_amdgcn_ballot_w64(stale) == 0) break;
+                                if (budget-- == 0u) {
+                                    ok = false;
+                                    break;
+                                }
+                                __builtin_amdgcn_s_sleep(1);
+                            }
+                            auto extra = [&](int i) -> uint32_t {
+                                return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m), i));
+                            };
+                            y = y_step(y, extra(1), static_cast<int32_t>(static_cast<uint32_t>(v)));
+                            z = z_step(z, extra(1));
+                            add(static_cast<uint32_t>(sum), extra(0), wave ? extra(4) : extra(2),
+                                wave ? extra(5) : extra(3));
+                        }
+                    }
+                }
+            }
+            if (!ok && lane == 0) sh.redo = 1u;
+        }
+        __syncthreads();
+        if (uniform(sh.redo) != 0u) {
+            // Run the whole head here, in order: scores, coefficients, Y and Z.
+            const int blocks = (pos + kBlock - 1) / kBlock;
+            for (int blk = wave; blk < blocks; blk += kWaves) {
+                load_k(pg, blk * kBlock, true, kb);
+                (void)take_scores(blk, 0, pos);
+            }
+            __syncthreads();
+            int32_t max_before = wave_scan_max(lane < blocks ? sh.blk_max[lane] : INT32_MIN);
+            top = __builtin_amdgcn_readlane(max_before, 63);
+            max_before = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, max_before);
+            for (int blk = wave; blk < blocks; blk += kWaves)
+                (void)take_words(blk, 0, pos, __builtin_amdgcn_readlane(max_before, blk), true);
+            __syncthreads();
+            if (wave < 2) {
+                const uint32_t word = coef_word(sh.new_score, top, sh.lut);
+                y = y_step(run_in_order(pg, sh, 0, d, 0, pos, 0), word, new_v);
+                z = z_step(z_in_order(sh, 0, lane, 0, pos, 0u), word);
             }
         }
     }
-    // The normalizer 1/Z: the 18-bit quotient floor((2^34 + Z/2) / Z) (cpp:271-300).
-    if (wave == 3 && lane == 0)
-        s_inv = z ? static_cast<uint32_t>(((1ull << 34) + (z >> 1)) / z) & 0x3ffffu : 0x3ffffu;
-    __syncthreads();
 
-    // Y * inv with RNE and a 32-bit wrap (cpp:1666-1710),
-    // and the integer-path A14/E8M0 (cpp:1694-1771, 2656-2682): group max of
-    // |raw| (INT32_MIN counts as INT32_MAX), one float conversion, frexp
-    // exponent e, q = trunc(clamp(raw*2^-17 * 2^(13-e) +- 0.5, +-8191)),
-    // code = e + 127.  Threads d < kCh own channel slice * kCh + d; a group
-    // is 32 lanes of one wave.
-    const size_t grp0 = static_cast<size_t>(b) * (kHeads * kGroupsPerHead) + h * kGroupsPerHead + slice * kGroups;
-    if (d < kCh) {
-        const int32_t o = mulq17_wrap(y, s_inv);
-        reinterpret_cast<int32_t*>(a.out)[static_cast<size_t>(b) * kModelDim + h * kHeadDim + slice * kCh + d] = o;
+    // Y * 1/Z with the 18-bit quotient floor((2^34 + Z/2) / Z) (cpp:271-300),
+    // RNE and a 32-bit wrap (cpp:1666-1710), and the integer-path A14/E8M0
+    // (cpp:1694-1771, 2656-2682): group max of |raw| (INT32_MIN counts as
+    // INT32_MAX), one float conversion, frexp exponent e, q =
+    // trunc(clamp(raw*2^-17 * 2^(13-e) +- 0.5, +-8191)), code = e + 127.
+    const size_t grp0 = static_cast<size_t>(b) * (kHeads * kGroupsPerHead) + h * kGroupsPerHead;
+    if (wave < 2) {
+        const uint32_t inv = z ? static_cast<uint32_t>(((1ull << 34) + (z >> 1)) / z) & 0x3ffffu : 0x3ffffu;
+        const int32_t o = mulq17_wrap(y, inv);
+        tail.out[static_cast<size_t>(b) * kModelDim + h * kHeadDim + d] = o;
         int32_t m = o == INT32_MIN ? INT32_MAX : (o < 0 ? -o : o);
 #pragma unroll
         for (int s = 1; s < 32; s <<= 1) m = max(m, __shfl_xor(m, s));
@@ -835,42 +1249,70 @@ __global__ __launch_bounds__(256) void exact_kernel(ExactArgs ea) {
             q14 = static_cast<int16_t>(static_cast<int>(rr));
             code = static_cast<uint8_t>(e + 127);
         }
-        s_q14[d] = q14;
-        if (a.act_scale != nullptr && (d & 31) == 0) a.act_scale[grp0 + (d >> 5)] = code;
+        sh.q14[d] = q14;
+        if (tail.act_scale != nullptr && (d & 31) == 0) tail.act_scale[grp0 + (d >> 5)] = code;
     }
     __syncthreads();
-    if (a.act_q != nullptr && d < kGroups * 14) {
+    if (tail.act_q != nullptr && d < kGroupsPerHead * 14) {
         const int gi = d / 14, w = d % 14;
         uint32_t word = 0;
         const int bit0 = 32 * w;
         for (int i = bit0 / 14; i <= (bit0 + 31) / 14 && i < 32; ++i) {
-            const uint32_t val = static_cast<uint32_t>(static_cast<uint16_t>(s_q14[gi * 32 + i])) & 0x3fffu;
-            const int sh = 14 * i - bit0;
-            word |= sh >= 0 ? (val << sh) : (val >> -sh);
+            const uint32_t val = static_cast<uint32_t>(static_cast<uint16_t>(sh.q14[gi * 32 + i])) & 0x3fffu;
+            const int shl = 14 * i - bit0;
+            word |= shl >= 0 ? (val << shl) : (val >> -shl);
         }
-        reinterpret_cast<uint32_t*>(a.act_q + (grp0 + gi) * 56)[w] = word;
+        reinterpret_cast<uint32_t*>(tail.act_q + (grp0 + gi) * 56)[w] = word;
+    }
+    if (SPLIT && !whole) {
+        // Every split's words have been read: advance the generation (and
+        // clear the head's slots when the tags wrap, so that no word left from
+        // 2^32-1 launches ago can pass for a current one).
+        if (tag == 0xffffffffu)
+            for (int i = d; i < nsplit * kExactSlotWords; i += kThreads)
+                __hip_atomic_store(slots + i, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (d == 0)
+            __hip_atomic_store(arrival, static_cast<uint64_t>(tag == 0xffffffffu ? 0u : tag) << 32, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!more) break;
+    // Nothing of this head is read from LDS any more but q14, which the next
+    // one writes behind further barriers.
+    h = next_h;
+    b = next_b;
+    pos = next_pos;
+    pg.rsrc = next.rsrc;
     }
 }
 
 }  // namespace
 
-hipError_t launch_exact(const StepArgs& a, const uint32_t* exp_lut, bool q17, hipStream_t s) {
-    ExactArgs ea;
-    ea.step = a;
-    for (int i = 0; i < 33; ++i) ea.exp_lut[i] = exp_lut[i];
-    if (a.batch <= kExactSlicedMaxBatch) {
-        const dim3 grid(kHeads * 4, a.batch);
-        if (q17) exact_kernel<true, 4><<<grid, 256, 0, s>>>(ea);
-        else exact_kernel<false, 4><<<grid, 256, 0, s>>>(ea);
-    } else if (a.batch <= kExactHalfSlicedMaxBatch) {
-        const dim3 grid(kHeads * 2, a.batch);
-        if (q17) exact_kernel<true, 2><<<grid, 256, 0, s>>>(ea);
-        else exact_kernel<false, 2><<<grid, 256, 0, s>>>(ea);
+hipError_t launch_exact(const StepArgs& a, int grid_splits, int cus, bool q17, hipStream_t s) {
+    if (a.split_tokens <= 0 || a.split_tokens % kSplitQuantum != 0 || a.split_tokens > kExactMaxTokens ||
+        a.kv.seq_cap > kMaxSeq || a.kv.layers > 0xffff || a.batch < 1 || a.batch > kMaxBatchPerLaunch || cus < 1 ||
+        grid_splits < 1 || (grid_splits > 1 && grid_splits > exact_splits(a.batch)))
+        return hipErrorInvalidValue;
+    StepPreload p = step_preload(a);
+    // Unsplit launches: one workgroup per CU (LDS holds no second one) takes
+    // heads in turn, back and forth over the rows (longest first), so that a
+    // ragged batch ends evenly.
+    const int rows = std::min({a.batch, std::max(cus / kHeads, 1), 255});   // of 32 workgroups
+    if (grid_splits == 1)
+        p.dispatch = (p.dispatch & StepPreload::kRowsListed) | static_cast<uint32_t>(a.batch - 1) << 16 |
+                     static_cast<uint32_t>(rows) << 24;
+    const dim3 grid = grid_splits > 1 ? dim3(grid_splits, kHeads, a.batch) : dim3(rows * kHeads);
+    const void* workspace = a.partials;
+#define SKV_EXACT(Q17, SPLIT)                                                                                        \
+    exact_kernel<Q17, SPLIT><<<grid, kThreads, 0, s>>>(p.layer_pages, p.geometry, p.dispatch, a.q, a.k, a.v, a.lut, \
+                                                       workspace, a)
+    if (grid_splits > 1) {
+        if (q17) SKV_EXACT(true, true);
+        else SKV_EXACT(false, true);
     } else {
-        const dim3 grid(kHeads, a.batch);
-        if (q17) exact_kernel<true, 1><<<grid, 256, 0, s>>>(ea);
-        else exact_kernel<false, 1><<<grid, 256, 0, s>>>(ea);
+        if (q17) SKV_EXACT(true, false);
+        else SKV_EXACT(false, false);
     }
+#undef SKV_EXACT
     return hipGetLastError();
 }
 

@@ -133,8 +133,9 @@ int swiftkv_debug_step_plan(int32_t cus, int32_t workgroups_per_cu, int32_t spli
  * workspace (noalloc = 0) or of this device's allocation-free workspace
  * (noalloc != 0) to `generation` and zeroes its partial words, on the context
  * stream, so a test can run launches across the wrap without 2^32 of them.
- * A context with no split workspace yet is left as it is (its first one
- * starts at generation 0).  Buffers the context keeps only for graphs that
+ * With noalloc = 0 it does the same to the integer-compatibility entry's
+ * exchange.  A context with no split workspace yet is otherwise left as it is
+ * (its first one starts at generation 0).  Buffers the context keeps only for graphs that
  * recorded them (see the graph section) are not reached.  `generation`
  * 0xffffffff is refused (SWIFTKV_EINVAL), and so is a call during graph
  * capture (SWIFTKV_ESTATE). */
@@ -142,7 +143,9 @@ int swiftkv_debug_set_split_generation(swiftkv_context* ctx, uint32_t generation
 /* Testing aid with no counterpart in the reference.  While enabled, every split
  * merge of the context's step launches waits for a tag that no partial carries,
  * so it gives up after one poll: the merged heads' outputs hold NaN and the
- * failure is reported as above.  Every kernel still exits normally and the
+ * failure is reported as above.  The integer-compatibility entry's results stay
+ * exact (a head whose splits' exchange gives up is run whole by one of them),
+ * and nothing is reported.  Every kernel still exits normally and the
  * split workspace stays consistent, so steps after it is disabled are exact
  * again.  Host-only; affects launches enqueued while it is on. */
 int swiftkv_debug_force_merge_timeout(swiftkv_context* ctx, int32_t enable);

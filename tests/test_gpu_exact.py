@@ -10,9 +10,11 @@ bit for bit:
     Q15.17 state, A14 words and E8M0 codes;
   - the reference's bound: positions at or past 4096 are refused.
 
-The kernel runs one of three launch shapes by batch size: four workgroups per
-(sequence, head) for batches 1-2, two for batches 3-8, one from batch 9.  The
-large-query, rescale-chain and saturation cases run in each shape."""
+Launches of up to 4 sequences split a head over 8, 4 or 2 workgroups (256
+tokens or more each) that exchange maxima and sums; larger ones give a
+workgroup whole heads, several in turn past 8 sequences; short sequences past 8
+take a kernel of their own.  The large-query, rescale-chain and saturation
+cases run in each."""
 import sys
 
 import numpy as np
@@ -107,9 +109,9 @@ def test_exact_matches_reference_decode(skv, ctx, lut4096, golden, case):
     ([1500, 77], "t3", True, False),
     ([300, 700], "wide", False, False),
     ([300, 700, 5, 257, 256, 511, 1, 0, 64], "wide", False, False),
-    ([300, 1030, 1], "normal", False, True),   # two workgroups per head
-    ([700], "t3", False, True),                # four workgroups per head
-    ([300, 1030, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),   # one workgroup per head
+    ([300, 1030, 1], "normal", False, True),   # split two ways
+    ([700], "t3", False, True),                # split three ways
+    ([300, 1030, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),   # whole heads, two turns
 ])
 def test_exact_matches_oracle_integer_recurrence(skv, ctx, lut4096, rope_tables, positions, dist, q17, big_query):
     """big_query: queries past 64.0 in some heads (and saturated channels in
@@ -153,7 +155,7 @@ def test_exact_matches_oracle_integer_recurrence(skv, ctx, lut4096, rope_tables,
     kv.close()
 
 
-@pytest.mark.parametrize("batch", [1, 3, 9])   # four, two and one workgroups per head
+@pytest.mark.parametrize("batch", [1, 3, 9])   # split heads, and short sequences' kernel
 def test_exact_every_token_a_new_maximum(skv, ctx, lut4096, rope_tables, batch):
     """Keys that grow along the query's direction make most tokens a new
     running maximum (578 of 700: INT8 quantization makes some neighbours tie,
@@ -206,7 +208,7 @@ def saturation_cases(mag, batch):
     return [cases[b % len(cases)] for b in range(batch)]
 
 
-# batch 1: four workgroups per head; 3: two; 9: one
+# batch 1 and 3: split heads; 9: whole heads in turn
 @pytest.mark.parametrize("mag,batch", [(31.0, 1), (31.0, 3), (31.0, 9), (40.0, 1), (40.0, 3), (40.0, 9)])
 def test_exact_y_saturates(skv, ctx, lut4096, rope_tables, mag, batch):
     """Y reaches INT32_MAX and INT32_MIN (alternate channels) early in a chunk
@@ -309,12 +311,12 @@ def test_exact_batch_over_one_launch(skv, ctx, lut4096, rope_tables):
 
 
 @pytest.mark.parametrize("batch,dist,outliers,q17", [(1, 0, True, False), (4, 1, False, True), (12, 0, False, False)],
-                         ids=["batch1_four_workgroups", "batch4_two_workgroups_t3", "batch12_one_workgroup"])
+                         ids=["batch1_split8", "batch4_split2_t3", "batch12_whole_heads"])
 def test_exact_position4095_matches_oracle(skv, ctx, lut4096, rope_tables, batch, dist, outliers, q17):
     """The integer-compatibility entry at the reference's last position, 4095
-    (16 chunks of 256 tokens per head), in each launch shape: four workgroups
-    per head (batch 1, K with 1% of channels x20), two (batch 4, Student-t(3),
-    Q15.17 inputs) and one (batch 12).  The device fills the cache from
+    (64 blocks of 64 tokens per head), split eight ways (batch 1, K with 1% of
+    channels x20), two ways (batch 4, Student-t(3), Q15.17 inputs) and whole
+    (batch 12).  The device fills the cache from
     synthetic streams through the append rule; the oracle rebuilds two sampled
     sequences from the same streams and runs the integer recurrence over all
     32 heads: every cached row, the appended row, the Q15.17 state, the A14
@@ -474,3 +476,125 @@ def test_host_io_mode_matches_device_mode(skv, ctx, lut4096, positions):
             assert all((x == y).all() for x, y in zip(got, want)), f"seq {b} head {h}"
     kv.close()
     kvh.close()
+
+
+def check_against_oracle(skv, ctx, lut, rope_tables, positions, dist, seed, step=None):
+    """One step on histories of `dist`, every sequence against the oracle's integer recurrence bit for bit."""
+    cos, sin = rope_tables
+    B = len(positions)
+    kv = skv.KVCache(ctx, layers=1, max_batch=B, max_seq_len=max(positions) + 1)
+    scs = []
+    for b, p in enumerate(positions):
+        kh, vh = history(seed + 10 * b, p, dist)
+        prefill(skv, ctx, kv, lut, 0, b, kh, vh)
+        scs.append(oracle_sequence(cos, sin, kh, vh, p + 1))
+    q = rising_query(B) if dist == "rising" else f32_normal(seed + 1000, (B, 4096))
+    k = rising_keys(positions) if dist == "rising" else f32_normal(seed + 1001, (B, 4096))
+    v = f32_normal(seed + 1002, (B, 4096))
+    qq, kq, vq = O.f2q17(q), O.f2q17(k), O.f2q17(v)
+    out, aq, asc = (step or exact_step)(skv, ctx, kv, lut, 0, positions, qq, kq, vq, q17=True)
+    for b, p in enumerate(positions):
+        res = scs[b].step_q17(qq[b], kq[b], vq[b], p, cos[p], sin[p], fp=False, integer=True)
+        assert_rows_equal(kv, scs[b], b, 0, p, 1)
+        ref = res["int"].reshape(4096)
+        diff = np.flatnonzero(out[b] != ref)
+        assert diff.size == 0, f"seq {b} position {p}: {diff.size} Q15.17 values differ (first {diff[:4]})"
+        q14, e8 = O.a14_q17(ref.reshape(128, 32))
+        assert (asc[b] == e8).all() and (aq[b] == O.pack_a14(q14)).all(), f"seq {b}: A14"
+    kv.close()
+
+
+@pytest.mark.parametrize("positions,dist", [
+    ([256], "normal"),                                           # a split of the new token alone
+    ([2047, 2048], "t3"),                                        # 4 splits of 512 and 768 tokens
+    ([900], "rising"),                                           # more new maxima than a split publishes
+    ([769, 0, 1, 63, 64, 65, 128, 1025, 448, 1100], "normal"),   # whole heads, two turns, one of no cached token
+    ([800, 511, 1000, 64, 900, 700, 1, 300, 769], "wide"),       # V shifts up to 25, in every term form
+    ([1000] * 9, "rising"),                                      # more accumulators than a workgroup holds
+    ([767, 0, 255, 256, 257, 511, 512, 1, 64], "normal"),        # the kernel for short sequences, at its bound
+    ([1279] + [40] * 16, "t3"),
+    ([1280] + [40] * 16, "t3"),
+])
+def test_exact_launch_forms(skv, ctx, lut4096, rope_tables, positions, dist):
+    """Each way a launch is cut up, at the edges of blocks, splits, turns and the rule between the two kernels."""
+    _note(f"case: exact launch forms, positions {positions}, {dist}")
+    check_against_oracle(skv, ctx, lut4096, rope_tables, positions, dist, 61000 + positions[0])
+
+
+@pytest.mark.parametrize("batch", [2, 5])   # split heads, and whole ones
+def test_exact_flat_attention(skv, ctx, lut4096, rope_tables, batch):
+    """Keys near zero, so every coefficient is near 1.0 and Z reaches 2,400, under V of 1, 6, 40 and 200 per
+    block of 1024 channels: sums whose bounds stay below the int32 range whole, cut at every eighth block of
+    tokens, cut at every block, and not even then (those run token by token)."""
+    _note(f"case: exact, flat attention, batch {batch}")
+    cos, sin = rope_tables
+    positions = [2400 - 700 * (b % 2) for b in range(batch)]
+    kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=max(positions) + 1)
+    mags = np.repeat(np.float32([1.0, 6.0, 40.0, 200.0]), 1024)
+    scs = []
+    for b, p in enumerate(positions):
+        kh, vh = history(63000 + 10 * b, p)
+        kh, vh = (kh * np.float32(0.01)).astype(np.float32), (vh * mags).astype(np.float32)
+        prefill(skv, ctx, kv, lut4096, 0, b, kh, vh)
+        scs.append(oracle_sequence(cos, sin, kh, vh, p + 1))
+    qq, kq, vq = (O.f2q17(f32_normal(63500 + i, (batch, 4096)) * np.float32([1, 0.01, 1][i])) for i in range(3))
+    out, aq, asc = exact_step(skv, ctx, kv, lut4096, 0, positions, qq, kq, vq, q17=True)
+    for b, p in enumerate(positions):
+        ref = scs[b].step_q17(qq[b], kq[b], vq[b], p, cos[p], sin[p], fp=False, integer=True)["int"].reshape(4096)
+        diff = np.flatnonzero(out[b] != ref)
+        assert diff.size == 0, f"seq {b} position {p}: {diff.size} Q15.17 values differ (first {diff[:4]})"
+    kv.close()
+
+
+def test_exact_split_that_hears_nothing(skv, ctx, lut4096, rope_tables):
+    """With every wait of the exchange giving up after one poll, no split learns of the maxima before it and no
+    sum is used: the last of a head to arrive runs all of it by itself, and the results are the same."""
+    _note("case: exact, exchange waits give up")
+
+    def step(*args, **kw):
+        ctx.debug_force_merge_timeout(True)
+        try:
+            return exact_step(*args, **kw)
+        finally:
+            ctx.debug_force_merge_timeout(False)
+
+    check_against_oracle(skv, ctx, lut4096, rope_tables, [1300], "normal", 62000, step)
+    check_against_oracle(skv, ctx, lut4096, rope_tables, [1300], "normal", 62000)
+
+
+def test_exact_repeats_bit_for_bit(skv, ctx, lut4096):
+    """1,000 launches of a split step, across the wrap of the exchange's tags, and replays of one captured before
+    any split step of its context, give the first launch's bits."""
+    _note("case: exact, 1000 launches across the tag wrap, and a graph")
+    p = 2500
+    with skv.Context(0) as other:
+        lut = skv.RopeLut.generate(other, 4096)
+        kv = skv.KVCache(other, layers=1, max_batch=1, max_seq_len=p + 1)
+        kv.fill_synthetic(lut, ntok=p, seed=71)
+        q, k, v = (other.to_device(f32_normal(7200 + i, (1, 4096))) for i in range(3))
+        out = other.alloc(4096 * 4)
+        other.capture_begin()
+        skv.swiftkv_attention_exact(other, q, k, v, kv, lut, None, None, 0, p, out)
+        graph = other.capture_end()
+        want = None
+        for turn in range(3):
+            graph.launch()
+            other.synchronize()
+            got = out.download(np.int32, (4096,))
+            want = got if want is None else want
+            assert (got == want).all(), f"replay {turn}"
+            out.zero()
+            skv.swiftkv_attention_exact(other, q, k, v, kv, lut, None, None, 0, p, out)
+            other.synchronize()
+            assert (out.download(np.int32, (4096,)) == want).all()
+        graph.close()
+        other.debug_set_split_generation(0xfffffe00)
+        for i in range(1000):
+            skv.swiftkv_attention_exact(other, q, k, v, kv, lut, None, None, 0, p, out)
+            if i % 50 == 49 or 505 <= i <= 520:
+                other.synchronize()
+                assert (out.download(np.int32, (4096,)) == want).all(), f"launch {i}"
+        for buf in (q, k, v, out):
+            buf.free()
+        kv.close()
+        lut.close()
