@@ -37,21 +37,27 @@ __device__ __forceinline__ int32_t mulq17_wrap(int32_t a, uint32_t b) {
 }
 
 // exp(x) for x <= 0 in Q1.17 through the 33-entry Q30 exp2 table with 12-bit
-// linear interpolation (swiftkv_attention.cpp:185-260).
+// linear interpolation (swiftkv_attention.cpp:185-260).  The reference's steps
+// with what cannot happen for x <= 0 left out, equal to them for every such x:
+//   - l = RNE(x log2(e) 2^-21) in its 24 bits: the product has at most 54
+//     significant bits, of which those past the 44 that x > -32.0 needs only
+//     decide that the result is 0, so the double product rounds as the integer
+//     one wherever that matters, and l > -2^23 there;
+//   - below -32.0 the shift is past 31 and the result 0, as the rule has it
+//     (both checked against the rule over every x above -40.0);
+//   - x = 0 gives l = 0 and 2^17, the shift is at least 13, and the result fits
+//     18 bits.
 __device__ __forceinline__ uint32_t exp_neg_q17(int32_t x, const uint32_t* lut) {
-    if (x >= 0) return 1u << 17;
-    if (x <= -(32 << 17)) return 0u;
-    const int64_t l = wrap_bits(rne_shift(static_cast<int64_t>(x) * kLog2eQ21, 21), 24);
-    const int64_t ex = l >> 17;
-    const uint32_t f = static_cast<uint32_t>(l - (ex << 17));
+    int32_t l;   // a saturating conversion
+    asm("v_cvt_i32_f64 %0, %1"
+        : "=v"(l)
+        : "v"(__builtin_rint(static_cast<double>(x) * (static_cast<double>(kLog2eQ21) * 0x1p-21))));
+    const uint32_t f = static_cast<uint32_t>(l) & 0x1ffffu;
     const uint32_t idx = f >> 12, rm = f & 0xfffu;
     const uint32_t base = lut[idx], next = lut[idx + 1];
     const uint32_t interp = base + static_cast<uint32_t>((static_cast<uint64_t>(next - base) * rm + (1u << 11)) >> 12);
-    const int sh = 13 - static_cast<int>(ex);
-    uint64_t out = 0;
-    if (sh <= 0) out = static_cast<uint64_t>(interp) << (-sh);
-    else if (sh < 32) out = (static_cast<uint64_t>(interp) + (1ull << (sh - 1))) >> sh;
-    return static_cast<uint32_t>(out) & 0x3ffffu;
+    const int sh = 13 - (l >> 17);
+    return sh < 32 ? (interp + (1u << ((sh - 1) & 31))) >> (sh & 31) : 0u;
 }
 
 // 44-bit token dot contribution of one 16-channel half-group, scaled by
@@ -75,9 +81,8 @@ constexpr uint32_t kMask30 = (1u << 30) - 1u;
 
 // Coefficient word of a token with score s and prefix maximum `before`.
 __device__ __forceinline__ uint32_t coef_word(int32_t s, int32_t before, const uint32_t* lut) {
-    const bool raise = s > before;
-    const int64_t x = raise ? static_cast<int64_t>(before) - s : static_cast<int64_t>(s) - before;
-    return exp_neg_q17(sat32(x), lut) | (raise ? kRescale : 0u);
+    const int32_t x = __builtin_elementwise_sub_sat(min(s, before), max(s, before));
+    return exp_neg_q17(x, lut) | (s > before ? kRescale : 0u);
 }
 
 // Z in Q13.17, wrapped to 30 bits.
