@@ -790,12 +790,20 @@ __global__ __launch_bounds__(WAVES * 64) void step_kernel(const int8_t* layer_pa
 // Prefill rows: one instruction covers two token rows (lane l takes channels
 // 4(l & 31) .. 4(l & 31) + 3 of row l >> 5), and a wave takes kAppendPairs
 // such pairs with all of their loads in flight together.  One pair per wave
-// and default-policy k/v loads measured fastest: more pairs per wave cost
-// occupancy, and nontemporal loads lose the MALL hits of k/v that a
-// projection has just written.
+// measured fastest: more pairs per wave cost occupancy.  k and v are read once,
+// with nontemporal loads: they still hit what a projection has just written into
+// the MALL and displace none of it, while default-policy loads push lines that
+// are still to be read out of it.  4095 tokens, us per call, default against
+// nontemporal: k and v just written by another kernel 36.0 against 29.4; written
+// before 400 MB of other data 50.8 against 34.4; read from HBM 35.4 against
+// 33.9; 1024 tokens 11.2 against 10.8; 333 tokens even.  (Only the same k and v
+// appended over and over, which the reads themselves keep in the MALL, is faster
+// with the default policy: 25.1 against 33.3.)  The rows are stored with the
+// default policy: nontemporal stores are 3-5% faster here (28.1), but a step
+// that follows then reads the rows from HBM (append and step 41.0 against 39.9).
 constexpr int kAppendPairs = 1;
 constexpr int kAppendTokens = 2 * kAppendPairs;
-constexpr bool kAppendNontemporal = false;
+constexpr bool kAppendNontemporal = true;
 
 // Q15.17 of four FP32 values by the saturating conversion alone, which maps
 // NaN to 0; the caller sends a wave holding a NaN through f32_to_q17.
