@@ -1,7 +1,7 @@
 // swiftkv_device.hpp -- device-side arithmetic shared by the kernels:
 // FP32 -> Q15.17, integer RoPE, G32 quantization, the append of one row, and
-// the DPP cross-lane helpers.  Included by swiftkv_kernels.hip and
-// swiftkv_synth.hip only.
+// the DPP cross-lane helpers.  Included by the .hip files and
+// swiftkv_exact.hpp only.
 #pragma once
 
 #include "swiftkv_common.hpp"
