@@ -986,11 +986,15 @@ __global__ __launch_bounds__(256) void append_bulk_kernel(const void* k_in, cons
 }
 
 // out[i] = Q15.17 of in[i] (NP = 1) or of the NP reduced split-K partials.
+// `stride` is the launch's thread count: it and the workgroup size, a constant,
+// are not read from the dispatch's own argument block, a scalar round trip ahead
+// of the first load and another at the loop's end.  Eight integer
+// steps of 5 rows with 4 partials, three conversions each: 282.9 us with those
+// reads, 282.1 without.
 template <int NP>
 __global__ __launch_bounds__(256) void convert_kernel(const float* __restrict__ in, int64_t part_stride,
-                                                      int32_t* __restrict__ out, size_t n) {
-    const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
-    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
+                                                      int32_t* __restrict__ out, size_t n, uint32_t stride) {
+    for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < n; i += stride) {
         if constexpr (NP == 1) {
             out[i] = f32_to_q17(in[i]);
         } else {
@@ -1116,9 +1120,9 @@ hipError_t launch_convert(const float* in, int32_t parts, int64_t part_stride, i
     if (blocks > 65536) blocks = 65536;
     const unsigned g = static_cast<unsigned>(blocks);
     switch (parts) {
-    case 1: convert_kernel<1><<<g, 256, 0, s>>>(in, part_stride, out, n); break;
-    case 2: convert_kernel<2><<<g, 256, 0, s>>>(in, part_stride, out, n); break;
-    case 4: convert_kernel<4><<<g, 256, 0, s>>>(in, part_stride, out, n); break;
+    case 1: convert_kernel<1><<<g, 256, 0, s>>>(in, part_stride, out, n, g * 256u); break;
+    case 2: convert_kernel<2><<<g, 256, 0, s>>>(in, part_stride, out, n, g * 256u); break;
+    case 4: convert_kernel<4><<<g, 256, 0, s>>>(in, part_stride, out, n, g * 256u); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
