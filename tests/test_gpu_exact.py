@@ -508,6 +508,7 @@ def check_against_oracle(skv, ctx, lut, rope_tables, positions, dist, seed, step
     ([256], "normal"),                                           # a split of the new token alone
     ([2047, 2048], "t3"),                                        # 4 splits of 512 and 768 tokens
     ([900], "rising"),                                           # more new maxima than a split publishes
+    ([464, 464, 1100], "wide"),                                  # split heads with V shifts of 16 and more
     ([769, 0, 1, 63, 64, 65, 128, 1025, 448, 1100], "normal"),   # whole heads, two turns, one of no cached token
     ([800, 511, 1000, 64, 900, 700, 1, 300, 769], "wide"),       # V shifts up to 25, in every term form
     ([1000] * 9, "rising"),                                      # more accumulators than a workgroup holds
