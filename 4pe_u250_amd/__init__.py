@@ -67,6 +67,7 @@ _SIGNATURES = {
     "swiftkv_synchronize": (C.c_int, [_vp]),
     "swiftkv_set_split_tokens": (C.c_int, [_vp, _i32]),
     "swiftkv_debug_set_split_generation": (C.c_int, [_vp, C.c_uint32, _i32]),
+    "swiftkv_debug_exchange_words": (C.c_int, [_vp, C.POINTER(C.c_int64)]),
     "swiftkv_debug_force_merge_timeout": (C.c_int, [_vp, _i32]),
     "swiftkv_debug_set_step_shape": (C.c_int, [_vp, _i32, _i32]),
     "swiftkv_debug_step_plan": (C.c_int, [_i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _vp, _vp]),
@@ -247,6 +248,12 @@ class Context:
         context's, or with noalloc this device's allocation-free one) and zero
         its partial words, so launches can be run across the tag wrap."""
         _check(lib().swiftkv_debug_set_split_generation(self.handle, int(generation), 1 if noalloc else 0))
+
+    def debug_exchange_words(self) -> int:
+        """Testing aid: words of the integer step's split exchange that hold anything."""
+        held = C.c_int64()
+        _check(lib().swiftkv_debug_exchange_words(self.handle, C.byref(held)))
+        return held.value
 
     def debug_force_merge_timeout(self, enable: bool) -> None:
         """Testing aid: while enabled, every split merge of this context's step

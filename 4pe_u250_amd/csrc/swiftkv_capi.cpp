@@ -16,6 +16,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -943,6 +944,20 @@ int swiftkv_debug_set_split_generation(swiftkv_context* ctx, uint32_t generation
     const size_t arrivals = arrival_words(rows);
     SKV_HIP(launch_fill_u64(base, arrivals, static_cast<uint64_t>(generation) << 32, ctx->stream));
     SKV_HIP(launch_fill_u64(base + arrivals, workspace_words(rows, slots) - arrivals, 0, ctx->stream));
+    return ok();
+}
+
+int swiftkv_debug_exchange_words(swiftkv_context* ctx, int64_t* held) {
+    if (!ctx || !held) return fail(SWIFTKV_EINVAL, "null argument");
+    int rc = not_capturing(ctx, "swiftkv_debug_exchange_words");
+    if (rc) return rc;
+    if ((rc = set_device(ctx))) return rc;
+    constexpr size_t first = kExactTableWords + kExactArrivalWords, n = kExactWorkspaceWords - first;
+    const std::unique_ptr<uint64_t[]> words(new (std::nothrow) uint64_t[n]);
+    if (!words) return fail(SWIFTKV_ENOMEM, "no host memory for %zu words", n);
+    SKV_HIP(hipStreamSynchronize(ctx->stream));
+    SKV_HIP(hipMemcpy(words.get(), ctx->exact_workspace + first, n * sizeof(uint64_t), hipMemcpyDeviceToHost));
+    *held = static_cast<int64_t>(n) - std::count(words.get(), words.get() + n, uint64_t(0));
     return ok();
 }
 

@@ -1269,10 +1269,11 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     }
     if (SPLIT && !whole) {
         // Every split's words have been read: advance the generation (and
-        // clear the head's slots when the tags wrap, so that no word left from
+        // clear all of the head's slots when the tags wrap, those of splits
+        // that only longer launches have among them, so that no word left from
         // 2^32-1 launches ago can pass for a current one).
         if (tag == 0xffffffffu)
-            for (int i = d; i < nsplit * kExactSlotWords; i += kThreads)
+            for (int i = d; i < exact_row_slots(b) * kExactSlotWords; i += kThreads)
                 __hip_atomic_store(slots + i, uint64_t(0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (d == 0)
             __hip_atomic_store(arrival, static_cast<uint64_t>(tag == 0xffffffffu ? 0u : tag) << 32, __ATOMIC_RELAXED,

@@ -140,6 +140,11 @@ int swiftkv_debug_step_plan(int32_t cus, int32_t workgroups_per_cu, int32_t spli
  * 0xffffffff is refused (SWIFTKV_EINVAL), and so is a call during graph
  * capture (SWIFTKV_ESTATE). */
 int swiftkv_debug_set_split_generation(swiftkv_context* ctx, uint32_t generation, int32_t noalloc);
+/* Testing aid with no counterpart in the reference: how many words of the
+ * integer-compatibility entry's exchange (all heads, without their arrival
+ * words) hold anything.  Synchronizes the context stream; refused during graph
+ * capture (SWIFTKV_ESTATE). */
+int swiftkv_debug_exchange_words(swiftkv_context* ctx, int64_t* held);
 /* Testing aid with no counterpart in the reference.  While enabled, every split
  * merge of the context's step launches waits for a tag that no partial carries,
  * so it gives up after one poll: the merged heads' outputs hold NaN and the

@@ -599,3 +599,24 @@ def test_exact_repeats_bit_for_bit(skv, ctx, lut4096):
             buf.free()
         kv.close()
         lut.close()
+
+
+def test_exact_tag_wrap_clears_every_split(skv, ctx, lut4096):
+    """A head whose tags wrap in a launch of few splits leaves no word of an earlier launch of more splits: such a
+    word would pass for a current one when its tag recurs."""
+    _note("case: exact, the tags wrap in a launch of fewer splits than the one before")
+    kv = skv.KVCache(ctx, layers=1, max_batch=2, max_seq_len=4096)
+    kv.fill_synthetic(lut4096, ntok=4095, seed=72)
+    q, k, v = (ctx.to_device(f32_normal(7300 + i, (2, 4096))) for i in range(3))
+    out = ctx.alloc(2 * 4096 * 4)
+    for longest, last in (([4095], [600]), ([4095, 4095], [300, 300])):
+        ctx.debug_set_split_generation(0xfffffffd)   # tag 0xfffffffe, then 0xffffffff, the last before the wrap
+        assert ctx.debug_exchange_words() == 0
+        skv.swiftkv_attention_exact(ctx, q, k, v, kv, lut4096, None, None, 0, longest, out)
+        assert ctx.debug_exchange_words() > 0
+        skv.swiftkv_attention_exact(ctx, q, k, v, kv, lut4096, None, None, 0, last, out)
+        assert ctx.debug_exchange_words() == 0, f"words of {longest} are left behind {last}"
+    ctx.debug_set_split_generation(0)
+    for buf in (q, k, v, out):
+        buf.free()
+    kv.close()
