@@ -11,7 +11,7 @@
 //     on neither; while no partial sum of Y can reach an end of the int32 range
 //     the saturating adds are plain adds, and a sum modulo 2^32 in any order is
 //     the reference's.  Each sum carries a bound of its terms' magnitudes; where
-//     |Y| plus the bound could reach 2^31 the segment is run token by token.
+//     |Y| plus the bound could reach 2^31 the range goes through the ordered pass.
 //
 // One 8-wave workgroup per CU.  Launches that split heads have the grid
 // (splits, 32 heads, batch rows); workgroup (j, h, z) owns tokens [j*C,
@@ -41,26 +41,41 @@
 // and the last of a head to arrive folds them (the fast step's exchange).  A
 // split that cannot publish in full -- it did not hear of the maxima before it
 // in time, or has too many new ones -- says so, and then, or where a bound
-// fails, the last to arrive runs the whole head by itself: no wait is
-// unbounded and no result depends on who waits for whom.
+// fails, the last to arrive runs the head from that split on by itself: no wait
+// is unbounded and no result depends on who waits for whom.
 //
-// What bounds it: for small batches the chain of round trips (first loads 3 us,
-// K pass 3, exchange of maxima 1.3, V pass 3.5, fold 1-4, exchange of sums 3);
-// for large ones the stream, at 6.9 TB/s within the K and V passes of a head,
-// with about 7 us of fold, barriers and ramps per 50 us head.  Context 4096,
-// us per call, the chunked kernel it replaced (Y in token order through LDS, up
-// to four workgroups per head each scoring every token) against this one: batch
-// 1 88.7 / 25.0, 2 92.2 / 30.6, 4 89.3 / 40.4, 8 111.8 / 58.8, 16 135.2 / 112.3,
-// 64 429.6 / 391.4; context 1536 at batch 5 52.1 / 27.5.  Tried: two 8-wave
-// workgroups per CU (128 registers, 480 at batch 64: their streams get in each
-// other's way, and a batch-1 launch then doubles workgroups up on half the CUs,
-// 39 against 28); reloading each row as soon as it is used (426 against 431, but
-// the compiler gives the rows other registers in each loop and waits for all
-// loads to copy them); sums per piece between new maxima (a masked pass and a
-// reduction each, 5-6 us per head more).  Only a head whose every token is a new
-// maximum is slower than before (batch 32: 1992 against 538): its hot blocks
-// outrun the staging rows and run from the page in order.
+// The ordered pass takes what the sums cannot carry, token by token: hot blocks
+// past the staging rows, ranges where a sum could saturate Y, splits with too
+// many new maxima.  Heads of rising scores (recency, drift) depend on it, so all
+// eight waves work at it: five stage terms in LDS while three run Y and Z over
+// the round before.
+//
+// What bounds it: for small batches the chain of round trips (first loads, K
+// pass, exchange of maxima, V pass, fold, exchange of sums); for large ones the
+// stream, at 6.9 TB/s within the K and V passes of a head, with about 7 us of
+// fold, barriers and ramps per 50 us head.  Calls back to back on one set of
+// buffers, context 4096, N(0, 1), us per call, the chunked kernel it replaced (Y
+// in token order through LDS, up to four workgroups per head each scoring every
+// token) against this one:
+//   batch     1           2           4           8          16          32         64
+//   normal    90.7 / 23.7 93.7 / 26.8 87.4 / 36.7 112 / 55.0 134 / 103   230 / 196  431 / 379
+//   scores that rise by 8 sigma over the last 200 tokens:
+//             103 / 36.3  109 / 46.5  100 / 71.6  121 / 59.4 145 / 111   239 / 214  442 / 411
+//   every token a new maximum:
+//             556 / 114   558 / 118   518 / 129   543 / 139  583 / 269   633 / 535  1242 / 1043
+// Slower than that kernel, which took every token from LDS at one rate: Y that
+// saturates for thousands of tokens, from batch 16 on (140 / 189; 435 / 717 at
+// 64), and scores that drift by 16 sigma and more over the context, from batch
+// 32 on (458 / 485 at 64; 271 / 319 at 64 and context 2048).
+// Tried: two 8-wave workgroups per CU (128 registers, 480 at batch 64: their
+// streams get in each other's way, and a batch-1 launch then doubles workgroups
+// up on half the CUs, 39 against 28);
+// reloading each row as soon as it is used (426 against 431, but the compiler
+// gives the rows other registers in each loop and waits for all loads to copy
+// them); sums per piece between new maxima (a masked pass and a reduction each,
+// 5-6 us per head more).
 #include <algorithm>
+#include <type_traits>
 
 #include "swiftkv_exact.hpp"
 
@@ -126,27 +141,40 @@ __device__ __forceinline__ uint32_t uniform(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v)));
 }
 
+__device__ __forceinline__ int8_t* uniform(int8_t* p) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    return reinterpret_cast<int8_t*>(static_cast<uint64_t>(uniform(static_cast<uint32_t>(v >> 32))) << 32 |
+                                     uniform(static_cast<uint32_t>(v)));
+}
+
 // ---------------------------------------------------------------- state
 
 struct Shared {
     // Per token of the range: x is the score, then the coefficient as a float
     // (sign set for a first or rescaling token, zero past the range); y the
     // biased exponents of the token's four V scales, a byte each.
-    uint2 tok[kExactMaxTokens];
+    uint2 tok[kExactMaxTokens + 2];               // and one that adds nothing, for the ordered pass
     // Sums of ordinary terms, modulo 2^32, of the coefficients, and of
     // coefficient times scale per group (the bound).
     int32_t pool[kPool][kHeadDim];
     uint32_t pool_z[kPool];
-    float pool_b[kPool][kGroupsPerHead];
+    __attribute__((aligned(16))) float pool_b[kPool][kGroupsPerHead];
     // Folding workgroups, per hot block: its tokens from the first to the last
     // special one, {first token | past the last << 16, row of `stage` where
     // they start (not staged if they would end past it), what Y is multiplied
-    // by at the first}; per staged token what Y is multiplied by (1.0 for an
-    // ordinary one) and what is added.
+    // by at the first}; per staged token what Y is multiplied by (Q1.17, 1.0 for
+    // an ordinary one; a float in the ordered pass) and what is added to it and
+    // to Z.
     uint4 hot[kPool];
-    uint32_t stage_mult[kStageRows];
+    __attribute__((aligned(16))) uint32_t stage_mult[kStageRows];
     int32_t stage[kStageRows][kHeadDim];
+    __attribute__((aligned(16))) int32_t stage_z[kStageRows];
+    // The ordered pass: its rows (tokens, or stretches as kSumRow | index), and
+    // per staged row the bounds of a stretch's sum.
+    uint16_t order[kExactMaxTokens + kMaxBlocks + 8];
+    __attribute__((aligned(16))) float stage_b[kStageRows][kGroupsPerHead];
     uint32_t staged;                              // rows taken so far
+    uint32_t unbounded;                           // a sum could saturate Y
     // Special (first or rescaling) tokens of a split that cannot fold its own
     // sums; number i uses pool entry kPool-1-i for the ordinary tokens after
     // it in its block.  Per hot block: its first special token and their count.
@@ -167,9 +195,10 @@ struct Shared {
     uint32_t failed;                              // the range's sums are incomplete
     uint32_t z;                                   // Z over the range
     uint32_t new_word;                            // the new token's coefficient word
-    uint32_t redo;                                // the splits' sums cannot be used
     uint32_t last;
-    uint32_t misc[16];                            // the split's own count and words of entries 0 and 1
+    uint32_t misc[16];                            // the split's own maximum, count and words of entries 0 and 1
+    uint32_t fail_at[2];                          // per folding wave: the first split whose sums cannot be used
+    int32_t max_before[kExactMaxSplits];          // running maximum before each split
     int16_t q14[kHeadDim];
 };
 
@@ -190,6 +219,20 @@ struct Page {
     int32_t scale_lane;      // lane's scale pair
     int32_t v_plane, s_plane, end;
 };
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t page_rsrc(int8_t* page, int cap) {
+    return __builtin_amdgcn_make_buffer_rsrc(page, static_cast<short>(0), cap * kTokenBytes, kBufferWord3);
+}
+__device__ __forceinline__ Page make_page(__amdgpu_buffer_rsrc_t rsrc, int cap, int c, int r) {
+    Page pg;
+    pg.rsrc = rsrc;
+    pg.code_lane = r * kCodeBytes + c * 16;
+    pg.scale_lane = r * kScaleBytes + (c >> 1) * 8;
+    pg.v_plane = cap * kCodeBytes;
+    pg.s_plane = cap * 2 * kCodeBytes;
+    pg.end = cap * kTokenBytes;
+    return pg;
+}
 
 constexpr int kNontemporal = 2;
 
@@ -258,6 +301,44 @@ __device__ __forceinline__ int32_t score_block(const KBlock& kb, const QueryLimb
     v_exp = static_cast<int32_t>(vs >> 23);
     const int32_t score = score_of((general >> c) & 1u ? own_i : static_cast<int64_t>(own_f));   // of token 8 c + r
     return __shfl(score, 8 * (lane & 7) + (lane >> 3));
+}
+
+// The scores of block `blk` of the range [first, end) into its tokens, and its
+// largest score and V scale; whether it has a V shift of 16 or more.
+__device__ __forceinline__ bool take_scores(const KBlock& kb, const QueryLimbs& ql, bool q3, Shared& sh, int blk,
+                                            int first, int end, int c, int r, int lane) {
+    uint2* const tok = sh.tok + blk * kBlock;
+    int32_t v_exp;
+    const int32_t score = score_block(kb, ql, q3, sh, tok, c, r, lane, v_exp);
+    tok[lane].x = static_cast<uint32_t>(score);
+    const int32_t mx = wave_scan_max(first + blk * kBlock + lane < end ? score : INT32_MIN);
+    v_exp = wave_scan_max(v_exp);
+    if (lane == 63) {
+        sh.blk_max[blk] = mx;
+        sh.blk_exp[blk] = v_exp;
+    }
+    return __builtin_amdgcn_readlane(v_exp, 63) >= static_cast<int32_t>(__float_as_uint(kWideScale) >> 23);
+}
+
+// The coefficient words of a block's tokens (lane = token) from their scores;
+// `start` is the running maximum before the block, which holds a new one if
+// is_hot.
+__device__ __forceinline__ uint32_t take_words(Shared& sh, int blk, int first, int end, int32_t start, bool is_hot,
+                                               int lane) {
+    uint2* const tok = sh.tok + blk * kBlock;
+    const bool valid = first + blk * kBlock + lane < end;
+    const int32_t score = static_cast<int32_t>(tok[lane].x);
+    int32_t pm = start;                            // running maximum before the lane's token
+    if (is_hot) {
+        pm = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, wave_scan_max(valid ? score : INT32_MIN));
+        pm = lane == 0 ? start : max(pm, start);
+    }
+    const bool init = first + blk + lane == 0;
+    const uint32_t word = !valid ? 0u : init ? kInit : coef_word(score, pm, sh.lut);
+    tok[lane].x = __float_as_uint(static_cast<float>(word & kCoefMask)) |
+                  ((word & (kInit | kRescale)) != 0u ? 0x80000000u : 0u);
+    wave_lds_sync();
+    return word;
 }
 
 // A wave's running sums of ordinary terms: per lane 16 channels of chunk c
@@ -383,8 +464,10 @@ __device__ __forceinline__ void flush(Shared& sh, int e, Sums& s, int lane) {
 // Where |y| plus the bound of a segment's terms stays below 2^31 no partial
 // sum saturates.  The bound: |code| <= 128, half a unit of rounding per term
 // and the roundings of the float sums.
+constexpr float kReach = 2147483000.0f;
+__device__ __forceinline__ float bound_reach(float b) { return b * 128.125f + 8192.0f; }
 __device__ __forceinline__ bool bounded(int32_t y, float b) {
-    return __builtin_fabsf(static_cast<float>(y)) + (b * 128.125f + 8192.0f) < 2147483000.0f;
+    return __builtin_fabsf(static_cast<float>(y)) + bound_reach(b) < kReach;
 }
 
 __device__ __forceinline__ uint32_t exps_shift(uint32_t exps, int g) { return ((exps >> (8 * g)) & 0xffu) - 110u; }
@@ -392,81 +475,63 @@ __device__ __forceinline__ uint32_t token_coef(uint32_t x) {
     return static_cast<uint32_t>(__builtin_fabsf(__uint_as_float(x)));
 }
 
-// Y of channel d over tokens [t0, t1) of the workgroup's range, in order, from
-// the coefficients in LDS and the V codes in the page.  `first` is the sequence
-// position of token 0 of the range.  Called by whole waves.
-__device__ __forceinline__ int32_t run_in_order(const Page& pg, const Shared& sh, int first, int d, int t0, int t1,
-                                                int32_t y) {
-    constexpr int kAhead = 8;
-    const int g = d >> 5;
-    const uint32_t rot = (9u + 8u * static_cast<uint32_t>(g)) & 31u;
-    int32_t next[kAhead];
-    auto load = [&](int t) {   // tokens past t1: in the page or zero, not used
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j)
-            next[j] = __builtin_amdgcn_raw_buffer_load_b8(pg.rsrc, d, pg.v_plane + (first + t + j) * kCodeBytes, 0);
-    };
-    load(t0);
-    for (int t = t0; t < t1; t += kAhead) {
-        int32_t code[kAhead];
-        uint2 w[kAhead];
-        uint32_t odd = 0, huge = 0;   // a special token or a shift of 16 or more; a shift of 24 or more
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) {
-            code[j] = static_cast<int8_t>(next[j]);
-            w[j] = sh.tok[min(t + j, t1 - 1)];
-            const uint32_t scale = __builtin_amdgcn_alignbit(w[j].y, w[j].y, rot) & 0x7f800000u;
-            odd |= (w[j].x >> 31) | static_cast<uint32_t>(scale >= __float_as_uint(kWideScale));
-            huge |= static_cast<uint32_t>(scale >= __float_as_uint(kHugeScale));
-        }
-        load(t + kAhead);
-        if (__builtin_amdgcn_ballot_w64(odd != 0u) == 0 && t + kAhead <= t1) {
-#pragma unroll
-            for (int j = 0; j < kAhead; ++j)
-                y = __builtin_elementwise_add_sat(
-                    y, static_cast<int32_t>(term_bits(code[j], token_product(w[j], rot)) - kRoundMagicBits));
-        } else if (__builtin_amdgcn_ballot_w64(huge != 0u) == 0 && t + kAhead <= t1) {
-            // Y = sat32(RNE(Y m >> 17) + x): m = 1.0 and x the term for an
-            // ordinary token, m the coefficient and x = v for a rescaling one,
-            // m = 0 and x = v for the first.
-            int32_t x[kAhead];
-            uint32_t m[kAhead];
-#pragma unroll
-            for (int j = 0; j < kAhead; ++j) {
-                const bool special = (w[j].x >> 31) != 0u;
-                m[j] = !special ? 1u << 17 : first + t + j == 0 ? 0u : token_coef(w[j].x);
-                uint2 wx = w[j];
-                if (special) wx.x = __float_as_uint(131072.0f);
-                x[j] = static_cast<int32_t>(__builtin_rintf(static_cast<float>(code[j]) * token_product(wx, rot)));
-            }
-#pragma unroll
-            for (int j = 0; j < kAhead; ++j) y = __builtin_elementwise_add_sat(mulq17_wrap(y, m[j]), x[j]);
-        } else {
+// Word of channel d in a staging row.  A lane writes 16 channels, four words at
+// a time: quad q of chunk c goes to word 4 (8 q + (c ^ 2 q)), so that eight
+// lanes write 128 bytes in a row (16 c + 4 q has four of them on each bank) and
+// the 32 channels of half a wave read from 32 banks.
+__device__ __forceinline__ int stage_quad(int c, int q) { return 4 * (8 * q + (c ^ (2 * q))); }
+__device__ __forceinline__ int stage_column(int d) { return stage_quad((d >> 4) & 7, (d >> 2) & 3) + (d & 3); }
+
+// Stages a token's terms for 16 channels: v itself for a special token (its
+// 2^17 scale = 2^shift), else the rounded product.  As the largest shift among
+// the tokens allows: one fused multiply-add (up to 15), a product and rint (up
+// to 23), 64-bit integers.
+enum TermForm { kTermFma, kTermRint, kTermAny };
+template <TermForm FORM>
+__device__ __forceinline__ void stage_row(int32_t* row, int c, v4i v, uint2 w, uint32_t rot) {
+    const uint32_t scale = __builtin_amdgcn_alignbit(w.y, w.y, rot) & 0x7f800000u;
+    const bool special = (w.x >> 31) != 0u;
+    if constexpr (FORM == kTermAny) {
+        const uint32_t coef = special ? 1u << 17 : token_coef(w.x);
 #pragma unroll 1
-            for (int j = 0; j < kAhead && t + j < t1; ++j) {
-                const uint2 wj = sh.tok[t + j];
-                int32_t x = code[0];
+        for (int q = 0; q < 4; ++q) {
+            v4i x;
 #pragma unroll
-                for (int i = 1; i < kAhead; ++i) x = i == j ? code[i] : x;
-                uint32_t word = token_coef(wj.x);
-                if ((wj.x >> 31) != 0u) word = first + t + j == 0 ? kInit : word | kRescale;
-                y = y_step(y, uniform(word), dequant_raw(x, exps_shift(wj.y, g)));
+            for (int j = 0; j < 4; ++j)
+                x[j] = mulq17_wrap(dequant_raw(static_cast<int8_t>(v[0] >> (8 * j)), (scale >> 23) - 110u), coef);
+            *reinterpret_cast<v4i*>(row + stage_quad(c, q)) = x;
+            v = __builtin_shufflevector(v, v, 1, 2, 3, 0);
+        }
+    } else {
+        const float p = (special ? 131072.0f : __uint_as_float(w.x)) * __uint_as_float(scale);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v4i x;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int32_t code = static_cast<int8_t>(v[q] >> (8 * j));
+                x[j] = FORM == kTermFma ? static_cast<int32_t>(term_bits(code, p) - kRoundMagicBits)
+                                        : static_cast<int32_t>(__builtin_rintf(static_cast<float>(code) * p));
             }
+            *reinterpret_cast<v4i*>(row + stage_quad(c, q)) = x;
         }
     }
-    return y;
 }
 
-// Y of channel d over `rows` staged tokens from row `at`.
-__device__ __forceinline__ int32_t run_staged(const Shared& sh, uint32_t at, int rows, int d, int32_t y) {
+// Y of a channel (its word `col` of a staging row), or Z (Z, every lane), over
+// `rows` (at most 64) staged tokens from row `at`.
+template <bool Z>
+__device__ __forceinline__ int32_t run_staged(const Shared& sh, uint32_t at, int rows, int col, int lane, int32_t y) {
     constexpr int kAhead = 8;
-    const int lane = d & 63;
     const uint32_t mult = lane < rows ? sh.stage_mult[at + static_cast<uint32_t>(lane)] : 1u << 17;
     const uint64_t special = __builtin_amdgcn_ballot_w64(mult != 1u << 17);
     int32_t next[kAhead];
     auto load = [&](int r) {
 #pragma unroll
-        for (int j = 0; j < kAhead; ++j) next[j] = sh.stage[at + static_cast<uint32_t>(min(r + j, rows - 1))][d];
+        for (int j = 0; j < kAhead; ++j) {
+            const uint32_t row = at + static_cast<uint32_t>(min(r + j, rows - 1));
+            next[j] = Z ? sh.stage_z[row] : sh.stage[row][col];
+        }
     };
     load(0);
     for (int r = 0; r < rows; r += kAhead) {
@@ -490,25 +555,250 @@ __device__ __forceinline__ int32_t run_staged(const Shared& sh, uint32_t at, int
     return y;
 }
 
-// Z over tokens [t0, t1), in order (one wave, lane = token): between special
-// tokens it advances by differences of prefix sums modulo 2^30.
-__device__ __forceinline__ uint32_t z_in_order(const Shared& sh, int first, int lane, int t0, int t1, uint32_t z) {
-    for (int t = t0; t < t1; t += 64) {
-        const uint32_t x = t + lane < t1 ? sh.tok[t + lane].x : 0u;
-        const uint32_t coef = token_coef(x);
-        uint64_t special = __builtin_amdgcn_ballot_w64((x >> 31) != 0u);
-        const int32_t incl = static_cast<int32_t>(wave_scan_add((x >> 31) != 0u ? 0u : coef));
-        uint32_t done = 0;
-        for (; special != 0u; special &= special - 1ull) {
-            const int i = __builtin_ctzll(special);
-            const uint32_t upto = static_cast<uint32_t>(__builtin_amdgcn_readlane(incl, i));
-            const uint32_t c = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(coef), i));
-            z = z_step((z + (upto - done)) & kMask30, first + t + i == 0 ? kInit : c | kRescale);
-            done = upto;
+// The ordered pass: Y and Z token by token, all waves at it, where sums do not
+// serve: hot blocks past the staging rows, stretches whose sum could saturate
+// Y, splits with more special tokens than entries.  It runs over a list of
+// rows, in rounds of 64: waves 4 to 7 gather the V codes of the rows' tokens
+// from the page, four rounds ahead, and stage their terms in one half of the
+// staging rows, and wave 3 what else the rows have; waves 0 and 1 take Y and
+// wave 2 takes Z over the other half.  LDS and the instructions of both sides
+// bound a round together: 0.7 us where every token adds a term, 1.25 where every
+// token rescales (0.3 the staging alone, 0.35 and 0.85 the fold alone).
+constexpr int kRound = kStageRows / 2;
+constexpr int kFetchAhead = 4;
+constexpr int kSumRow = 0x8000;
+constexpr float kNoBound = -1e9f;                 // of a row that is no sum
+
+// Y (or Z) over a staged round's rows from row `at` (those past the list's end
+// add nothing): sat32(RNE(Y m) + x).  A row goes through a double, three
+// dependent operations: the product (50 bits) plus 1.5 2^52 rounds once, to an
+// integer, to nearest even, and the low word is that integer.  In a loop alone,
+// from LDS: 13.3 ns a row; the 64-bit integer form 25.8, clamping in doubles
+// 18.8, rint and convert 16.7.  One straight path for the round: chosen every 8
+// rows, the taken branches cost more than the additions between them.
+// `worst`: the largest |Y| around a round's sums, plus their largest bound.
+template <bool Z>
+__device__ __forceinline__ int32_t run_round(const Shared& sh, int at, int d, int lane, int32_t y, float& worst) {
+    const int g = (d >> 5) & 3, col = stage_column(d);
+    int32_t x[kRound];
+    auto load = [&](int r) {
+#pragma unroll
+        for (int j = r; j < r + kRound / 2; ++j)
+            if (!Z) x[j] = sh.stage[at + j][col];
+    };
+    const int own = static_cast<int>(sh.stage_mult[at + lane]);   // of row `lane`
+    const int own_z = Z ? sh.stage_z[at + lane] : 0;
+    const float own_bound = sh.stage_b[at + lane][0];
+    load(0);
+    const bool special = __builtin_amdgcn_ballot_w64(own != __float_as_int(1.0f)) != 0u;
+    const uint64_t sums = Z ? 0u : __builtin_amdgcn_ballot_w64(own_bound != kNoBound);
+    load(kRound / 2);
+    auto term = [&](int j) { return Z ? __builtin_amdgcn_readlane(own_z, j) : x[j]; };
+    auto step = [&](int j) {
+        const float m = __int_as_float(__builtin_amdgcn_readlane(own, j));
+        const double t = __builtin_fma(static_cast<double>(y), static_cast<double>(m), 0x1.8p52);
+        y = __builtin_elementwise_add_sat(static_cast<int32_t>(__double2loint(t)), term(j));
+    };
+    if (Z && !special) {   // Z stays below 2^30: a sum in any order
+        y += __builtin_amdgcn_readlane(static_cast<int>(wave_scan_add(static_cast<uint32_t>(own_z))), 63);
+    } else if (sums == 0u && !special) {
+#pragma unroll
+        for (int j = 0; j < kRound; ++j) y = __builtin_elementwise_add_sat(y, term(j));
+    } else if (sums == 0u) {
+#pragma unroll
+        for (int j = 0; j < kRound; ++j) step(j);
+    } else {
+        float bound = kNoBound;
+        for (uint64_t s = sums; s != 0u; s &= s - 1ull) bound = fmaxf(bound, sh.stage_b[at + __builtin_ctzll(s)][g]);
+        int32_t hi = y, lo = y;
+#pragma unroll
+        for (int j = 0; j < kRound; ++j) {
+            step(j);
+            hi = max(hi, y);
+            lo = min(lo, y);
         }
-        z = (z + (static_cast<uint32_t>(__builtin_amdgcn_readlane(incl, 63)) - done)) & kMask30;
+        const int32_t most = max(hi, lo == INT32_MIN ? INT32_MAX : -lo);
+        worst = fmaxf(worst, static_cast<float>(most) + bound_reach(bound));
     }
-    return z;
+    return y;
+}
+
+__device__ __forceinline__ int round_barriers(int rounds) {
+    return (rounds + kFetchAhead - 1) / kFetchAhead * kFetchAhead;
+}
+
+// Waves 4 to 7: the terms of all rounds.
+template <TermForm FORM, bool PIECES>
+__device__ __forceinline__ void stage_rounds(__amdgpu_buffer_rsrc_t rsrc, Shared& sh, int cap, int first, int total,
+                                             int rounds, int wave, int lane) {
+    struct Fetched {
+        v4i v[2];
+        uint2 word[2];
+        int sum[2];                               // a sum's index, or -1
+    };
+    Fetched f[kFetchAhead];
+    const int c = lane & 7, mine = 8 * (wave - 4) + (lane >> 3);   // and 32 more
+    const uint32_t rot = (9u + 8u * static_cast<uint32_t>(c >> 1)) & 31u;
+    auto fetch = [&](int round, Fetched& x) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = round * kRound + mine + 32 * u;
+            const int row = PIECES ? static_cast<int>(sh.order[min(i, total - 1)]) : i;
+            const bool sum = PIECES && row >= kSumRow && i < total, none = sum || i >= total;
+            const int token = none ? 0 : row;
+            x.word[u] = sh.tok[none ? kExactMaxTokens : row];
+            x.sum[u] = sum ? row & (kSumRow - 1) : -1;
+            x.v[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (first + token) * kCodeBytes + 16 * c, cap * kCodeBytes, 0);
+        }
+    };
+    auto stage = [&](int round, const Fetched& x) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            int32_t* const to = sh.stage[(round & 1) * kRound + mine + 32 * u];
+            stage_row<FORM>(to, c, x.v[u], x.word[u], rot);
+            if (PIECES && x.sum[u] >= 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<v4i*>(to + stage_quad(c, q)) =
+                        reinterpret_cast<const v4i*>(&sh.pool[x.sum[u]][16 * c])[q];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < kFetchAhead; ++u) fetch(u, f[u]);
+    stage(0, f[0]);
+    fetch(kFetchAhead, f[0]);
+    // Barrier b hands round b to the folding waves.  The fetches are made on
+    // every path, so that the loads in flight stay countable.
+    for (int b = 0; b < round_barriers(rounds); b += kFetchAhead) {
+#pragma unroll
+        for (int u = 0; u < kFetchAhead; ++u) {
+            __syncthreads();
+            const int round = b + u + 1;
+            if (round < rounds) stage(round, f[(u + 1) % kFetchAhead]);
+            fetch(round + kFetchAhead, f[(u + 1) % kFetchAhead]);
+        }
+    }
+}
+
+// With `pieces` its rows are the tokens of the hot blocks' spans, and in front
+// of each span and after the last one the sum of the stretch there (where one
+// fails its bound sh.unbounded is set); without, tokens [0, count).  `first` is
+// the sequence position of token 0.  Returns Y (waves 0 and 1) or Z (wave 2)
+// from `y`.  Every wave makes the same number of barriers.
+//
+// Out of line, so that its registers are its own: inlined, the kernel's own
+// path spills, and took 26.0 us at batch 1 against 23.9.  Arguments arrive in vector registers; all but
+// y are wave-uniform.
+typedef __attribute__((address_space(3))) Shared* SharedPtr;
+__device__ __attribute__((noinline)) int32_t ordered_pass(int8_t* page, SharedPtr shared, int cap_arg, int first_arg,
+                                                          int count_arg, int pieces_arg, int nbound_arg, int32_t y) {
+    Shared& sh = *(Shared*)shared;
+    const int first = uniform(first_arg), count = uniform(count_arg);
+    const int nbound = uniform(nbound_arg), cap = uniform(cap_arg);
+    const bool pieces = uniform(pieces_arg) != 0;
+    const __amdgpu_buffer_rsrc_t rsrc = page_rsrc(uniform(page), cap);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, d = threadIdx.x;
+    int total = count;
+    if (pieces) {
+        const uint32_t span = lane < nbound ? sh.hot[lane].x : 0u;
+        const int32_t len = static_cast<int32_t>(span >> 16) - static_cast<int32_t>(span & 0xffffu);
+        const int32_t past = static_cast<int32_t>(wave_scan_add(lane < nbound ? static_cast<uint32_t>(len) + 1u : 0u));
+        total = __builtin_amdgcn_readlane(past, 63) + 1;
+        for (int k = wave; k < nbound; k += kWaves) {
+            const int n = __builtin_amdgcn_readlane(len, k), at = __builtin_amdgcn_readlane(past, k) - n;
+            const int token = __builtin_amdgcn_readlane(static_cast<int>(span), k) & 0xffff;
+            if (lane < n) sh.order[at + lane] = static_cast<uint16_t>(token + lane);
+            if (lane == 0) sh.order[at - 1] = static_cast<uint16_t>(kSumRow | k);
+        }
+        if (d == 0) sh.order[total - 1] = static_cast<uint16_t>(kSumRow | nbound);
+        __syncthreads();
+    }
+    const int rounds = (total + kRound - 1) / kRound;
+    const int barriers = round_barriers(rounds);
+    if (rounds == 0) return y;
+    if (wave >= 4) {
+        const int widest = __builtin_amdgcn_readlane(
+            wave_scan_max(lane < (count + kBlock - 1) / kBlock ? sh.blk_exp[lane] : 0), 63);
+        auto produce = [&](auto form) {
+            if (pieces) stage_rounds<form.value, true>(rsrc, sh, cap, first, total, rounds, wave, lane);
+            else stage_rounds<form.value, false>(rsrc, sh, cap, first, total, rounds, wave, lane);
+        };
+        if (widest >= static_cast<int>(__float_as_uint(kHugeScale) >> 23))
+            produce(std::integral_constant<TermForm, kTermAny>());
+        else if (widest >= static_cast<int>(__float_as_uint(kWideScale) >> 23))
+            produce(std::integral_constant<TermForm, kTermRint>());
+        else
+            produce(std::integral_constant<TermForm, kTermFma>());
+    } else if (wave == 3) {
+        auto describe = [&](int round) {          // lane = row
+            const int i = round * kRound + lane, at = (round & 1) * kRound + lane;
+            const int row = pieces ? static_cast<int>(sh.order[min(i, total - 1)]) : i;
+            const bool past = i >= total, sum = pieces && row >= kSumRow;
+            const uint32_t x = past || sum ? 0u : sh.tok[row].x;
+            const bool special = (x >> 31) != 0u;
+            const float coef = __builtin_fabsf(__uint_as_float(x));
+            float mult = special ? coef * 0x1p-17f : 1.0f;   // 0.0 for the sequence's first token
+            int32_t z = special ? 1 << 17 : static_cast<int32_t>(coef);
+            float4 bound = make_float4(kNoBound, kNoBound, kNoBound, kNoBound);
+            if (sum && !past) {
+                z = static_cast<int32_t>(sh.pool_z[row & (kSumRow - 1)]);
+                bound = *reinterpret_cast<const float4*>(sh.pool_b[row & (kSumRow - 1)]);
+            }
+            sh.stage_mult[at] = __float_as_uint(mult);
+            sh.stage_z[at] = z;
+            *reinterpret_cast<float4*>(sh.stage_b[at]) = bound;
+        };
+        describe(0);
+        for (int b = 0; b < barriers; ++b) {
+            __syncthreads();
+            if (b + 1 < rounds) describe(b + 1);
+        }
+    } else {
+        float worst = 0.0f;
+        __builtin_amdgcn_s_setprio(3);             // ahead of the staging wave on its SIMD
+        for (int b = 0; b < barriers; ++b) {
+            __syncthreads();
+            const int at = (b & 1) * kRound;
+            if (b < rounds) {
+                if (wave < 2) y = run_round<false>(sh, at, d, lane, y, worst);
+                else y = run_round<true>(sh, at, d, lane, y, worst);
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        if (!(worst < kReach)) sh.unbounded = 1u;
+    }
+    return y;
+}
+
+// Runs the head from token `first` on, in order, after the sums of the splits
+// before: scores, coefficients (the new token's too), then the ordered pass
+// from `y` (Y in waves 0 and 1, Z in wave 2).  Out of line like it.
+__device__ __attribute__((noinline)) int32_t run_rest(int8_t* page, SharedPtr shared, int cap_arg, int first_arg,
+                                                      int end_arg, int32_t max_before, QueryLimbs ql, int q3, int32_t y) {
+    Shared& sh = *(Shared*)shared;
+    const int cap = uniform(cap_arg), first = uniform(first_arg), end = uniform(end_arg), count = end - first;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int c = lane & 7, r = lane >> 3;
+    const Page pg = make_page(page_rsrc(uniform(page), cap), cap, c, r);
+    const int blocks = (count + kBlock - 1) / kBlock;
+    KBlock kb;
+    load_k(pg, first + wave * kBlock, wave < blocks, kb);
+    for (int blk = wave; blk < blocks; blk += kWaves) {
+        (void)take_scores(kb, ql, uniform(q3) != 0, sh, blk, first, end, c, r, lane);
+        load_k(pg, first + (blk + kWaves) * kBlock, blk + kWaves < blocks, kb);
+    }
+    __syncthreads();
+    const int32_t m = max(max_before, wave_scan_max(lane < blocks ? sh.blk_max[lane] : INT32_MIN));
+    int32_t before = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, m);
+    before = lane == 0 ? max_before : before;
+    for (int blk = wave; blk < blocks; blk += kWaves)
+        (void)take_words(sh, blk, first, end, __builtin_amdgcn_readlane(before, blk), true, lane);
+    if (wave == 0 && lane == 0) sh.new_word = coef_word(sh.new_score, __builtin_amdgcn_readlane(m, 63), sh.lut);
+    __syncthreads();
+    return ordered_pass(page, shared, cap, first, count, 0, 0, y);
 }
 
 // Tagged words of the split exchange: the launch's tag above a 32-bit value.
@@ -528,8 +818,8 @@ constexpr uint32_t kPrefixPolls = 256;
 // A split's slot: its maximum, then its entries.  Entry e holds the sums
 // A[128], the values V[128] of the special token they follow (none for entry
 // 0), and six words {z, word, bounds of the four groups}; those of entries 0
-// and 1 lie together behind the count, so that one load per split, a word per
-// lane, takes them.
+// and 1 lie together behind the maximum and the count, so that one load per
+// split, a word per lane, takes all of them.
 constexpr uint32_t kSlotFailed = 1u << 31;
 constexpr int kSlotMax = 0, kSlotCount = 1, kSlotMisc = 2, kSlotEntries = kSlotMisc + 6 * kExactEntries;
 static_assert(kExactSlotWords >= kSlotEntries + kExactEntries * 2 * kHeadDim, "slot layout");
@@ -579,19 +869,11 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     const bool owner = split == nsplit - 1;       // appends the new row
     const bool whole = nsplit == 1;
     const int begin = split * C;
-    Page pg;
-    pg.end = cap * kTokenBytes;
-    pg.v_plane = cap * kCodeBytes;
-    pg.s_plane = cap * 2 * kCodeBytes;
-    pg.code_lane = r * kCodeBytes + c * 16;
-    pg.scale_lane = r * kScaleBytes + (c >> 1) * 8;
     auto page_of = [&](int seq, int head) {
-        int8_t* const page = const_cast<int8_t*>(layer_pages) +
-                             (static_cast<int64_t>(seq) * (geometry >> 16) * kHeads + head) *
-                                 (static_cast<int64_t>(cap) * kTokenBytes);
-        return __builtin_amdgcn_make_buffer_rsrc(page, static_cast<short>(0), pg.end, kBufferWord3);
+        return const_cast<int8_t*>(layer_pages) + (static_cast<int64_t>(seq) * (geometry >> 16) * kHeads + head) *
+                                                      (static_cast<int64_t>(cap) * kTokenBytes);
     };
-    pg.rsrc = page_of(b, h);
+    Page pg = make_page(page_rsrc(page_of(b, h), cap), cap, c, r);
 
     // All loads of the prologue, then the first K and V blocks, before any math.
     int2 cs;
@@ -645,7 +927,7 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
         }
     }
     Page next = pg;
-    next.rsrc = page_of(next_b, next_h);
+    next.rsrc = page_rsrc(page_of(next_b, next_h), cap);
     const int32_t next_past = more && wave < blocks_of(next_pos) ? 0 : pg.end;
     for (int i = d; i < kPool * kHeadDim / 4; i += kThreads)
         reinterpret_cast<int4*>(&sh.pool[0][0])[i] = make_int4(0, 0, 0, 0);
@@ -654,8 +936,10 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
         *reinterpret_cast<float4*>(sh.pool_b[d]) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
     if (d == 0) {
+        sh.tok[kExactMaxTokens] = make_uint2(0u, 0u);
         sh.specials = 0u;
         sh.staged = 0u;
+        sh.unbounded = 0u;
         sh.failed = 0u;
     }
 
@@ -711,24 +995,11 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     // K pass.  Rows past `stop` are read (inside the page, or zero) and their
     // scores dropped.
     uint32_t wide_blocks = 0;                      // own blocks with a V shift of 16 or more
-    auto take_scores = [&](int blk, int first, int end) -> bool {
-        uint2* const tok = sh.tok + blk * kBlock;
-        int32_t v_exp;
-        const int32_t score = score_block(kb, ql, q3, sh, tok, c, r, lane, v_exp);
-        tok[lane].x = static_cast<uint32_t>(score);
-        const int32_t mx = wave_scan_max(first + blk * kBlock + lane < end ? score : INT32_MIN);
-        v_exp = wave_scan_max(v_exp);
-        if (lane == 63) {
-            sh.blk_max[blk] = mx;
-            sh.blk_exp[blk] = v_exp;
-        }
-        return __builtin_amdgcn_readlane(v_exp, 63) >= static_cast<int32_t>(__float_as_uint(kWideScale) >> 23);
-    };
     // (One place loads the blocks, also for a wave without any: with several
     // the compiler gives them different registers, and copying between those
     // waits for the loads.)
     for (int it = 0; it == 0 || it < own_blocks; ++it) {
-        if (own_blocks > 0 && take_scores(wave + it * kWaves, begin, stop)) wide_blocks |= 1u << it;
+        if (own_blocks > 0 && take_scores(kb, ql, q3, sh, wave + it * kWaves, begin, stop, c, r, lane)) wide_blocks |= 1u << it;
         const bool here = it + 1 < own_blocks;
         load_k(here ? pg : next, here ? begin + (wave + (it + 1) * kWaves) * kBlock : wave * kBlock,
                here || next_past == 0, kb);
@@ -751,7 +1022,10 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     int32_t before_range = INT32_MIN;
     if (SPLIT && !whole) {
         if (wave == 0) {
-            if (lane == 63) publish(mine + kSlotMax, tag, static_cast<uint32_t>(incl));
+            if (lane == 63) {
+                publish(mine + kSlotMax, tag, static_cast<uint32_t>(incl));
+                sh.misc[0] = static_cast<uint32_t>(incl);
+            }
             int32_t m = INT32_MIN;
             bool ok = true;
             if (lane < split) {
@@ -777,48 +1051,31 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     int32_t before = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, incl);
     before = lane == 0 ? before_range : max(before, before_range);
     const uint64_t hot = __builtin_amdgcn_ballot_w64(lane < nblk && (bm > before || (begin == 0 && lane == 0)));
-    // A stretch whose sum could saturate Y as far as its bound tells is run
-    // token by token, so where coefficients stay near 1.0 over many tokens of
-    // large V the stretches are cut, at every 8th block or at every block.
-    // Lane = block: 64 terms of at most 128 2^shift times the largest
-    // coefficient.
+    // A stretch whose sum could saturate Y as far as its bound tells sends the
+    // range through the ordered pass, so where coefficients stay near 1.0 over
+    // many tokens of large V the stretches are cut, so that the bound of each
+    // stays near 2^30.  Lane = block: 64 terms of at most 128 2^shift times the
+    // largest coefficient, and the cuts where their running sum passes multiples
+    // of 2^30.  (Batch 32, 4096 tokens, V scaled per token by e^(1.5 N(0, 1)):
+    // 262 us; with a cut at every block where eight could pass 2^30, 279.)
     uint64_t cuts = 0;
     {
         const float coef = fast_exp2((static_cast<float>(min(bm, before)) - static_cast<float>(before)) *
                                      (1.4426950408889634f * 0x1p-17f));
         const float most = lane < nblk ? ldexpf(coef, sh.blk_exp[lane] - 110 + 13) : 0.0f;
-        const float eight = octet_sum(most);
-        if (uniform(__float_as_int(across_octets_sum(eight))) >= __float_as_int(0x1p30f))
-            cuts = uniform(__float_as_int(across_octets_max(eight))) >= __float_as_int(0x1p30f) ? ~1ull : 0x0101010101010100ull;
-        if (nblk < 64) cuts &= (1ull << nblk) - 1ull;
+        const int32_t passed = static_cast<int32_t>(fminf(wave_scan_add(most) * 0x1p-30f, 1e6f));
+        cuts = __builtin_amdgcn_ballot_w64(lane > 0 && lane < nblk && passed != dpp_shifted<kDppWaveShr1, 0xF>(0, passed));
     }
     const uint64_t bounds = hot | cuts;            // where stretches end
     const int nbound = __builtin_popcountll(bounds);
-    int32_t top = max(before_range, __builtin_amdgcn_readlane(incl, 63));   // running maximum before the new token
+    const int32_t top = max(before_range, __builtin_amdgcn_readlane(incl, 63));   // running maximum before the new token
     // Whether the fold can start at the range's first token: a hot block is
-    // then run in order from its V codes (staged in LDS for the first few);
+    // then run in order from its terms (staged in LDS as far as they fit);
     // other splits sum the pieces between its special tokens.
     const bool folds = !SPLIT || split == 0;
     static_assert(kMaxBlocks + 1 + kSpecials <= kPool, "an accumulator per stretch and per special token");
 
-    // V pass.  First the coefficient words of a block's tokens (lane = token);
-    // `start` is the running maximum before the block.
-    auto take_words = [&](int blk, int first, int end, int32_t start, bool is_hot) -> uint32_t {
-        uint2* const tok = sh.tok + blk * kBlock;
-        const bool valid = first + blk * kBlock + lane < end;
-        const int32_t score = static_cast<int32_t>(tok[lane].x);
-        int32_t pm = start;                        // running maximum before the lane's token
-        if (is_hot) {
-            pm = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, wave_scan_max(valid ? score : INT32_MIN));
-            pm = lane == 0 ? start : max(pm, start);
-        }
-        const bool init = first + blk + lane == 0;
-        const uint32_t word = !valid ? 0u : init ? kInit : coef_word(score, pm, sh.lut);
-        tok[lane].x = __float_as_uint(static_cast<float>(word & kCoefMask)) |
-                      ((word & (kInit | kRescale)) != 0u ? 0x80000000u : 0u);
-        wave_lds_sync();
-        return word;
-    };
+    // V pass.  First the coefficient words of a block's tokens.
     const uint32_t rot = (9u + 8u * static_cast<uint32_t>(c >> 1)) & 31u;   // exponent byte c / 2 to bits 23..30
     Sums s;
     s.clear();
@@ -843,7 +1100,7 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
         stretch = k;
         const bool wide = (wide_blocks >> it) & 1u;
         const uint2* const tok = sh.tok + blk * kBlock;
-        const uint32_t word = take_words(blk, begin, stop, __builtin_amdgcn_readlane(before, blk), is_hot);
+        const uint32_t word = take_words(sh, blk, begin, stop, __builtin_amdgcn_readlane(before, blk), is_hot, lane);
         const uint32_t coef = word & kCoefMask;
         if (!is_hot) {
             s.z += coef;
@@ -852,46 +1109,36 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
             dirty = true;
         } else if (folds) {
             // From the first to the last special token the block is run in
-            // order later; the tokens before join the stretch that ends here,
-            // those after the next one.
+            // order later (by the ordered pass, where one block does not fit the
+            // staging rows); the tokens before join the stretch that ends
+            // here, those after the next one.
             const uint64_t m = __builtin_amdgcn_ballot_w64((word & (kInit | kRescale)) != 0u);
             const int t_first = __builtin_ctzll(m), t_last = 63 - __builtin_clzll(m);
             const int rows = t_last - t_first + 1;
-            uint32_t at = kStageRows;
             const uint2 own = tok[lane];
             const bool special = (own.x >> 31) != 0u;
             const uint32_t widest = max(max(own.y & 0xffu, (own.y >> 8) & 0xffu), max((own.y >> 16) & 0xffu, own.y >> 24));
             const bool huge = __builtin_amdgcn_ballot_w64(widest >= __float_as_uint(kHugeScale) >> 23) != 0;
-            if (!huge && lane == 0) at = atomicAdd(&sh.staged, static_cast<uint32_t>(rows));
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&sh.staged, huge ? kStageRows + 1u : static_cast<uint32_t>(rows));
             at = uniform(at);
             if (lane == t_first)
                 sh.hot[k] = make_uint4(static_cast<uint32_t>(blk * kBlock + t_first) |
                                            static_cast<uint32_t>(blk * kBlock + t_last + 1) << 16,
                                        at, (word & kInit) ? 0u : coef, 0u);
-            if (at + static_cast<uint32_t>(rows) <= static_cast<uint32_t>(kStageRows)) {
-                if (lane >= t_first && lane <= t_last)
-                    sh.stage_mult[at + static_cast<uint32_t>(lane - t_first)] =
-                        !special ? 1u << 17 : (word & kInit) ? 0u : coef;
+            if (!huge && at + static_cast<uint32_t>(rows) <= static_cast<uint32_t>(kStageRows)) {
+                if (lane >= t_first && lane <= t_last) {
+                    const uint32_t i = at + static_cast<uint32_t>(lane - t_first);
+                    sh.stage_mult[i] = !special ? 1u << 17 : (word & kInit) ? 0u : coef;
+                    sh.stage_z[i] = special ? 1 << 17 : static_cast<int32_t>(coef);
+                }
 #pragma unroll
                 for (int i = 0; i < kRows; ++i) {
                     const int t = 8 * i + r;
-                    uint2 w = tok[t];
-                    if ((w.x >> 31) != 0u) w.x = __float_as_uint(131072.0f);   // v itself: 2^17 scale = 2^shift
-                    const float p = token_product(w, rot);
                     v4i v = vb.v[i];
                     asm volatile("" : "+v"(v));   // as in add_wide_terms
-                    if (t >= t_first && t <= t_last) {
-                        v4i* const out = reinterpret_cast<v4i*>(&sh.stage[at + static_cast<uint32_t>(t - t_first)][16 * c]);
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            v4i x;
-#pragma unroll
-                            for (int j = 0; j < 4; ++j)
-                                x[j] = static_cast<int32_t>(__builtin_rintf(
-                                    static_cast<float>(static_cast<int8_t>(v[q] >> (8 * j))) * p));
-                            out[q] = x;
-                        }
-                    }
+                    if (t >= t_first && t <= t_last)
+                        stage_row<kTermRint>(sh.stage[at + static_cast<uint32_t>(t - t_first)], c, v, tok[t], rot);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
@@ -964,6 +1211,7 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     if (dirty) flush(sh, stretch, s, lane);
     __syncthreads();
     const bool usable = uniform(sh.failed) == 0u;
+    const bool staged = uniform(sh.staged) <= static_cast<uint32_t>(kStageRows);
 
     // The fold: the stretches' sums and the hot blocks in token order, one
     // thread per channel for Y, one wave for Z.
@@ -971,88 +1219,85 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
     int32_t y = 0;
     uint32_t z = 0;
     const int32_t new_v = dequant_raw(sh.new_code[d & (kHeadDim - 1)], exps_shift(sh.new_exps, g));
-    if (wave < 2 && folds) {
+    auto fold = [&](auto z_column) {
         // Stretch k, then hot block k's span, often one token; what block k + 1
         // needs is read ahead.
+        constexpr bool Z = decltype(z_column)::value;
+        const int col = stage_column(d);
         const uint4 table = sh.hot[lane];
         auto column = [&](uint32_t x, int k) {
             return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(x), k));
         };
-        const int n = usable ? nbound : 0;
-        int32_t sum = sh.pool[0][d], first = sh.stage[min(column(table.y, 0), kStageRows - 1u)][d];
-        float bound = sh.pool_b[0][g];
-        int from = 0;
+        auto sum_of = [&](int k) { return Z ? static_cast<int32_t>(sh.pool_z[k]) : sh.pool[k][d]; };
+        auto first_of = [&](int k) {
+            const uint32_t row = min(column(table.y, k & 63), kStageRows - 1u);
+            return Z ? sh.stage_z[row] : sh.stage[row][col];
+        };
+        int32_t sum = sum_of(0), first = first_of(0);
+        float bound = Z ? 0.0f : sh.pool_b[0][g];
         for (int k = 0;; ++k) {
             const int32_t sum_k = sum, first_k = first;
             const float bound_k = bound;
-            const int kn = min(k + 1, n);
-            sum = sh.pool[kn][d];
-            bound = sh.pool_b[kn][g];
-            first = sh.stage[min(column(table.y, kn & 63), kStageRows - 1u)][d];
-            const uint32_t span = column(table.x, k & 63), at = column(table.y, k & 63);
-            const int span0 = k < n ? static_cast<int>(span & 0xffffu) : stop - begin;
-            if (usable && __builtin_amdgcn_ballot_w64(!bounded(y, bound_k)) == 0) y += sum_k;
-            else y = run_in_order(pg, sh, begin, d, from, span0, y);
-            if (k == n) break;
-            from = static_cast<int>(span >> 16);
-            const int rows = from - span0;         // none at a cut
+            const int kn = min(k + 1, nbound);
+            sum = sum_of(kn);
+            if (!Z) bound = sh.pool_b[kn][g];
+            first = first_of(kn);
+            if (!Z && __builtin_amdgcn_ballot_w64(!bounded(y, bound_k)) != 0) {
+                if (lane == 0) sh.unbounded = 1u;
+                break;
+            }
+            y += sum_k;
+            if (k == nbound) break;
+            const uint32_t span = column(table.x, k), at = column(table.y, k);
+            const int rows = static_cast<int>(span >> 16) - static_cast<int>(span & 0xffffu);   // none at a cut
             if (rows == 0) continue;
-            if (at + static_cast<uint32_t>(rows) <= static_cast<uint32_t>(kStageRows)) {
-                y = __builtin_elementwise_add_sat(mulq17_wrap(y, column(table.z, k)), first_k);
-                if (rows > 1) y = run_staged(sh, at + 1u, rows - 1, d, y);
-            } else {
-                y = run_in_order(pg, sh, begin, d, span0, from, y);
-            }
+            y = __builtin_elementwise_add_sat(mulq17_wrap(y, column(table.z, k)), first_k);
+            if (rows > 1) y = run_staged<Z>(sh, at + 1u, rows - 1, col, lane, y);
         }
-    } else if (wave == 2) {
-        const uint32_t word = pos == 0 ? kInit : coef_word(sh.new_score, top, sh.lut);
-        if (folds) {
-            const uint4 table = sh.hot[lane];
-            const uint32_t zs = sh.pool_z[lane], z_last = sh.pool_z[64];
-            if (!usable) z = z_in_order(sh, begin, lane, 0, stop - begin, z);
-            for (int k = 0; usable; ++k) {
-                z = (z + (k < 64 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(zs), k)) : z_last)) &
-                    kMask30;
-                if (k == nbound) break;
-                const uint32_t span = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(table.x), k));
-                const uint32_t mult = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(table.z), k));
-                const int span0 = static_cast<int>(span & 0xffffu), span1 = static_cast<int>(span >> 16);
-                if (span0 == span1) continue;
-                z = z_step(z, begin + span0 == 0 ? kInit : mult | kRescale);
-                if (span0 + 1 < span1) z = z_in_order(sh, begin, lane, span0 + 1, span1, z);
-            }
-            if (whole) z = z_step(z, word);
-        }
-        if (lane == 0) {
-            sh.z = z;
-            sh.new_word = word;
-        }
+    };
+    if (folds && staged) {
+        if (wave < 2) fold(std::false_type());
+        else if (wave == 2) fold(std::true_type());
+    }
+    if (wave == 2 && lane == 0) {
+        sh.z = static_cast<uint32_t>(y);
+        sh.new_word = pos == 0 ? kInit : coef_word(sh.new_score, top, sh.lut);
     }
     __syncthreads();
-    z = sh.z;
-    const uint32_t new_word = uniform(sh.new_word);
-    if (whole && wave < 2) y = y_step(y, new_word, new_v);
+    uint32_t new_word = uniform(sh.new_word);
 
+    // Where that does not serve, the ordered pass over the range.
+    if (folds && (!staged || uniform(sh.unbounded) != 0u)) {
+        for (bool pieces = uniform(sh.unbounded) == 0u;; pieces = false) {
+            y = ordered_pass(page_of(b, h), (SharedPtr)&sh, cap, begin, stop - begin, pieces ? 1 : 0, nbound, 0);
+            if (wave == 2 && lane == 0) sh.z = static_cast<uint32_t>(y);
+            __syncthreads();
+            if (!pieces || uniform(sh.unbounded) == 0u) break;
+        }
+    }
+    z = sh.z;
+
+    bool add_new = true;                           // or the new token is in the merged sums
     if (SPLIT && !whole) {
         // Publish the range's entries; a split that cannot only says so.  Its own
-        // sums of entries 0 and 1 stay at hand, in case it is the one that folds.
-        uint32_t own_a0 = 0, own_a1 = 0, own_v1 = 0;
+        // entries 0 and 1 stay in LDS (sums in staging rows 0 and 1, values in
+        // row 2), in case it is the one that folds: in registers they end up in
+        // scratch memory, and reading that waits for the words just published.
         if (wave < 2) {
             int entries = 1;
             auto put = [&](int e, uint32_t av, uint32_t zv, float bv) {
                 publish(slot_sums(mine, e) + d, tag, av);
                 if (d == 0) publish(slot_misc(mine, e), tag, zv);
                 if ((d & 31) == 0) publish(slot_misc(mine, e) + 2 + g, tag, __float_as_uint(bv));
-                if (e == 0) own_a0 = av;
-                if (e == 1) own_a1 = av;
-                if (e < 2 && d == 0) sh.misc[1 + 6 * e] = zv;
-                if (e < 2 && (d & 31) == 0) sh.misc[3 + 6 * e + g] = __float_as_uint(bv);
+                if (e < 2) sh.stage[e][d] = static_cast<int32_t>(av);
+                if (e < 2 && d == 0) sh.misc[2 + 6 * e] = zv;
+                if (e < 2 && (d & 31) == 0) sh.misc[4 + 6 * e + g] = __float_as_uint(bv);
             };
             auto put_special = [&](int e, uint32_t word, int32_t v) {
                 publish(slot_values(mine, e) + d, tag, static_cast<uint32_t>(v));
                 if (d == 0) publish(slot_misc(mine, e) + 1, tag, word);
-                if (e == 1) own_v1 = static_cast<uint32_t>(v);
-                if (e < 2 && d == 0) sh.misc[2 + 6 * e] = word;
+                if (e == 1) sh.stage[2][d] = v;
+                if (e < 2 && d == 0) sh.misc[3 + 6 * e] = word;
             };
             if (folds) {
                 put(0, static_cast<uint32_t>(y), z, 0.0f);
@@ -1091,7 +1336,7 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
             }
             if (d == 0) {
                 publish(mine + kSlotCount, tag, static_cast<uint32_t>(entries));
-                sh.misc[0] = static_cast<uint32_t>(entries);
+                sh.misc[1] = static_cast<uint32_t>(entries);
             }
         }
         // The count goes out from a wave that publishes nothing.
@@ -1099,30 +1344,35 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
         if (threadIdx.x == kCountThread) {
             const uint64_t n = __hip_atomic_fetch_add(arrival, uint64_t(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             sh.last = static_cast<uint32_t>(n) == static_cast<uint32_t>(nsplit - 1);
-            sh.redo = 0u;
         }
         __syncthreads();
         if (!uniform(sh.last)) return;
 
         // The last split of the head to arrive folds the entries of all of
         // them.  Every split has counted, so its words land by themselves.
-        // Entries 0 and 1 of every split come in one round of loads.
+        // Entries 0 and 1 of every split come in one round of loads.  A wave
+        // stops at the first split whose sums cannot be used; pool holds Y, and
+        // pool_z Z, before each split.
         if (wave < 2) {
             bool ok = true;
             uint32_t budget = tail.merge_polls;
-            constexpr int kMisc = 13;              // the count and the words of entries 0 and 1
+            constexpr int kMisc = 14;              // the maximum, the count and the words of entries 0 and 1
+            const uint64_t own_tag = static_cast<uint64_t>(want) << 32;
+            const uint64_t own_m = own_tag | sh.misc[min(lane, kMisc - 1)];
+            const uint64_t own_a0 = own_tag | static_cast<uint32_t>(sh.stage[0][d]);
+            const uint64_t own_a1 = own_tag | static_cast<uint32_t>(sh.stage[1][d]);
+            const uint64_t own_v1 = own_tag | static_cast<uint32_t>(sh.stage[2][d]);
             uint64_t mw[kExactMaxSplits], a0[kExactMaxSplits], a1[kExactMaxSplits], v1[kExactMaxSplits];
             for (;;) {
 #pragma unroll
                 for (int j = 0; j < kExactMaxSplits; ++j) {
-                    const uint64_t own_tag = static_cast<uint64_t>(want) << 32;
-                    mw[j] = own_tag | sh.misc[min(lane, kMisc - 1)];
-                    a0[j] = own_tag | own_a0;
-                    a1[j] = own_tag | own_a1;
-                    v1[j] = own_tag | own_v1;
+                    mw[j] = own_m;
+                    a0[j] = own_a0;
+                    a1[j] = own_a1;
+                    v1[j] = own_v1;
                     if (j < nsplit && j != split) {
                         uint64_t* const p = slots + j * kExactSlotWords;
-                        mw[j] = fetch(p + kSlotCount + min(lane, kMisc - 1));
+                        mw[j] = fetch(p + kSlotMax + min(lane, kMisc - 1));
                         a0[j] = fetch(slot_sums(p, 0) + d);
                         a1[j] = fetch(slot_sums(p, 1) + d);
                         v1[j] = fetch(slot_values(p, 1) + d);
@@ -1132,15 +1382,15 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
 #pragma unroll
                 for (int j = 0; j < kExactMaxSplits; ++j) {
                     if (j < nsplit) {
-                        const uint64_t count = __builtin_amdgcn_readlane(static_cast<int>(mw[j] >> 32), 0) ==
+                        const uint64_t count = __builtin_amdgcn_readlane(static_cast<int>(mw[j] >> 32), 1) ==
                                                        static_cast<int>(want)
-                                                   ? uniform(static_cast<uint32_t>(mw[j]))
+                                                   ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mw[j]), 1))
                                                    : 0u;
-                        // of a failed split nothing but the count is read
+                        // of a failed split nothing but the maximum and the count is read
                         const bool failed = (count & kSlotFailed) != 0u, more = !failed && count > 1u;
                         stale |= count == 0u || (!failed && !current(a0[j], want)) ||
                                  (more && (!current(a1[j], want) || !current(v1[j], want))) ||
-                                 (!failed && lane >= 1 && lane < (more ? kMisc : 7) && lane != 2 &&
+                                 ((lane == 0 || (!failed && lane >= 2 && lane < (more ? kMisc : 8) && lane != 3)) &&
                                   !current(mw[j], want));
                     }
                 }
@@ -1151,15 +1401,30 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
                 }
                 __builtin_amdgcn_s_sleep(1);
             }
+            int fail_at = ok ? nsplit : 0;
+            int32_t max_before = INT32_MIN;
             y = 0;
             z = 0u;
+            sh.pool[0][d] = 0;
+            if (lane == 0) {
+                sh.pool_z[0] = 0u;
+                sh.max_before[0] = INT32_MIN;
+            }
 #pragma unroll
             for (int j = 0; j < kExactMaxSplits; ++j) {
                 if (j < nsplit && ok) {
+                    if (j > 0) {
+                        sh.pool[j][d] = y;
+                        if (lane == 0) {               // the same values from both waves
+                            sh.pool_z[j] = z;
+                            sh.max_before[j] = max_before;
+                        }
+                    }
                     auto misc = [&](int i) -> uint32_t {
                         return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mw[j]), i));
                     };
-                    const uint32_t n = misc(0);
+                    const uint32_t n = misc(1);
+                    max_before = max(max_before, static_cast<int32_t>(misc(0)));
                     auto add = [&](uint32_t sum, uint32_t coefs, uint32_t bound_lo, uint32_t bound_hi) {
                         const float bv = __uint_as_float((d & 32) ? bound_hi : bound_lo);
                         ok = ok && __builtin_amdgcn_ballot_w64(!bounded(y, bv)) == 0;
@@ -1169,12 +1434,12 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
                     if (n & kSlotFailed) {
                         ok = false;
                     } else {
-                        add(static_cast<uint32_t>(a0[j]), misc(1), wave ? misc(5) : misc(3), wave ? misc(6) : misc(4));
+                        add(static_cast<uint32_t>(a0[j]), misc(2), wave ? misc(6) : misc(4), wave ? misc(7) : misc(5));
                         if (n > 1) {
-                            y = y_step(y, misc(8), static_cast<int32_t>(static_cast<uint32_t>(v1[j])));
-                            z = z_step(z, misc(8));
-                            add(static_cast<uint32_t>(a1[j]), misc(7), wave ? misc(11) : misc(9),
-                                wave ? misc(12) : misc(10));
+                            y = y_step(y, misc(9), static_cast<int32_t>(static_cast<uint32_t>(v1[j])));
+                            z = z_step(z, misc(9));
+                            add(static_cast<uint32_t>(a1[j]), misc(8), wave ? misc(12) : misc(10),
+                                wave ? misc(13) : misc(11));
                         }
                         for (uint32_t e = 2; ok && e < n; ++e) {
                             uint64_t* const p = slots + j * kExactSlotWords;
@@ -1200,31 +1465,28 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
                                 wave ? extra(5) : extra(3));
                         }
                     }
+                    if (!ok) fail_at = j;
                 }
             }
-            if (!ok && lane == 0) sh.redo = 1u;
+            if (lane == 0) sh.fail_at[wave] = static_cast<uint32_t>(fail_at);
         }
         __syncthreads();
-        if (uniform(sh.redo) != 0u) {
-            // Run the whole head here, in order: scores, coefficients, Y and Z.
-            const int blocks = (pos + kBlock - 1) / kBlock;
-            for (int blk = wave; blk < blocks; blk += kWaves) {
-                load_k(pg, blk * kBlock, true, kb);
-                (void)take_scores(blk, 0, pos);
-            }
+        const int fail_at = static_cast<int>(min(uniform(sh.fail_at[0]), uniform(sh.fail_at[1])));
+        add_new = fail_at < nsplit;
+        if (add_new) {
+            const int32_t before = wave == 2 ? static_cast<int32_t>(sh.pool_z[fail_at])
+                                             : sh.pool[fail_at][d & (kHeadDim - 1)];
+            y = run_rest(page_of(b, h), (SharedPtr)&sh, cap, fail_at * C, pos, sh.max_before[fail_at], ql, q3 ? 1 : 0,
+                         before);
+            if (wave == 2 && lane == 0) sh.z = static_cast<uint32_t>(y);
             __syncthreads();
-            int32_t max_before = wave_scan_max(lane < blocks ? sh.blk_max[lane] : INT32_MIN);
-            top = __builtin_amdgcn_readlane(max_before, 63);
-            max_before = dpp_shifted<kDppWaveShr1, 0xF>(INT32_MIN, max_before);
-            for (int blk = wave; blk < blocks; blk += kWaves)
-                (void)take_words(blk, 0, pos, __builtin_amdgcn_readlane(max_before, blk), true);
-            __syncthreads();
-            if (wave < 2) {
-                const uint32_t word = coef_word(sh.new_score, top, sh.lut);
-                y = y_step(run_in_order(pg, sh, 0, d, 0, pos, 0), word, new_v);
-                z = z_step(z_in_order(sh, 0, lane, 0, pos, 0u), word);
-            }
+            z = sh.z;
+            new_word = uniform(sh.new_word);
         }
+    }
+    if (add_new) {
+        if (wave < 2) y = y_step(y, new_word, new_v);
+        z = z_step(z, new_word);
     }
 
     // Y * 1/Z with the 18-bit quotient floor((2^34 + Z/2) / Z) (cpp:271-300),

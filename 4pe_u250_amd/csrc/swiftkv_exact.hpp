@@ -171,5 +171,15 @@ __device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
     return static_cast<uint32_t>(x + dpp_shifted<kDppRowBcast31, 0xC>(0, x));
 }
 
+__device__ __forceinline__ float wave_scan_add(float v) {
+    auto from = [](float x, auto move) { return __int_as_float(move(__float_as_int(x))); };
+    v += from(v, [](int32_t x) { return dpp_shifted<kDppRowShr1, 0xF>(0, x); });
+    v += from(v, [](int32_t x) { return dpp_shifted<kDppRowShr2, 0xF>(0, x); });
+    v += from(v, [](int32_t x) { return dpp_shifted<kDppRowShr4, 0xF>(0, x); });
+    v += from(v, [](int32_t x) { return dpp_shifted<kDppRowShr8, 0xF>(0, x); });
+    v += from(v, [](int32_t x) { return dpp_shifted<kDppRowBcast15, 0xA>(0, x); });
+    return v + from(v, [](int32_t x) { return dpp_shifted<kDppRowBcast31, 0xC>(0, x); });
+}
+
 }  // namespace exact
 }  // namespace swiftkv

@@ -16,12 +16,13 @@ workgroup whole heads, several in turn past 8 sequences; short sequences past 8
 take a kernel of their own.  The large-query, rescale-chain and saturation
 cases run in each."""
 import sys
+import time
 
 import numpy as np
 import pytest
 
 import oracle as O
-from gpu_cases import (H, assert_rows_equal, history, oracle_cache_synthetic, oracle_sequence, outlier_channels,
+from gpu_cases import (H, RISING_CHANNELS, assert_rows_equal, history, oracle_cache_synthetic, oracle_sequence, outlier_channels,
                        prefill, rising_keys, rising_query)
 from helpers import f32_normal, kat_vector
 
@@ -620,3 +621,116 @@ def test_exact_tag_wrap_clears_every_split(skv, ctx, lut4096):
     for buf in (q, k, v, out):
         buf.free()
     kv.close()
+
+
+def biased_history(seed, n, bias, v_scale=1.0, v_dist="normal"):
+    """History whose scores against biased_query have bias(t) added, on channels too slow for the rotation to
+    undo it."""
+    k, v = history(seed, n, v_dist)
+    k[:, RISING_CHANNELS] = (bias(np.arange(n, dtype=np.float64)) / 0.7071)[:, None].astype(np.float32)
+    return k, (v * np.float32(v_scale)).astype(np.float32)
+
+
+def biased_query(seed, batch):
+    q = f32_normal(seed, (batch, 4096))
+    q[:, RISING_CHANNELS] = 1.0
+    return q
+
+
+BIASES = {
+    "tail": lambda n: lambda t: 6.0 * np.clip(1.0 - (n - t) / 200.0, 0.0, None),   # the last tokens win
+    "middle": lambda n: lambda t: 6.0 * np.exp(-np.abs(t - n / 2) / 60.0),
+    "drift": lambda n: lambda t: 16.0 * t / n,
+    "steep": lambda n: lambda t: 60.0 * t / n,
+}
+
+
+@pytest.mark.parametrize("positions,bias,v_scale,v_dist,first", [
+    ([1300], "tail", 1, "normal", 0),              # the last split's maxima do not fit its entries
+    ([1300], "middle", 1, "normal", 0),            # a split in the middle: it and those after it run in order
+    ([1500, 1200], "steep", 1, "normal", 0),       # every split but the first
+    ([320], "steep", 1, "normal", 0),              # the ordered pass over 64 tokens of the second split,
+    ([319], "steep", 1, "normal", 0),              # 63,
+    ([321], "steep", 1, "normal", 0),              # 65,
+    ([384], "steep", 1, "normal", 0),              # and 128: whole rounds and their edges
+    ([1400, 900, 1024, 1100, 64], "drift", 1, "normal", 0),   # whole heads: more hot rows than staging rows
+    ([1400, 900, 1024, 1100, 64], "steep", 1, "normal", 0),
+    ([1400, 900, 1024, 1100, 64], "drift", 30, "normal", 0),  # V shifts of 16 and more
+    ([1100, 900, 1024, 700, 64], "drift", 1, "wide", 0),      # and of 24 and more
+    ([1400, 900, 1300, 1100, 64], "drift", 300, "normal", 0), # sums that fail their bounds: the whole range in order
+    ([1300, 1100], "drift", 300, "normal", 0),
+    ([1300], "steep", 1, "normal", 100),           # tokens 0 to 99 never appended: zero codes and zero scales
+    ([1300] * 5, "steep", 1, "normal", 100),
+])
+def test_exact_ordered_pass(skv, ctx, lut4096, rope_tables, positions, bias, v_scale, v_dist, first):
+    """Heads whose scores rise: what the sums between new maxima cannot carry goes through the ordered pass, in
+    each of its forms, bit for bit as the oracle has it."""
+    _note(f"case: exact ordered pass, positions {positions}, {bias}, V x{v_scale} {v_dist}, first {first}")
+    cos, sin = rope_tables
+    batch, seed = len(positions), 64000 + positions[0]
+    kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=max(positions) + 1)
+    kv.zero()
+    scs = []
+    for b, p in enumerate(positions):
+        kh, vh = biased_history(seed + 10 * b, p, BIASES[bias](p), v_scale, v_dist)
+        at = first if p > first else 0
+        dk, dv = ctx.to_device(kh[at:]), ctx.to_device(vh[at:])
+        skv.swiftkv_append_tokens(ctx, dk, dv, kv, lut4096, 0, b, at, p - at)
+        ctx.synchronize()
+        dk.free()
+        dv.free()
+        scs.append(O.SequenceCache(H, p + 1))
+        scs[-1].fill_q17(O.f2q17(kh[at:]), O.f2q17(vh[at:]), at, cos, sin)
+    q = biased_query(seed + 1, batch)
+    k, v = f32_normal(seed + 2, (batch, 4096)), f32_normal(seed + 3, (batch, 4096))
+    qq, kq, vq = O.f2q17(q), O.f2q17(k), O.f2q17(v)
+    for forced in (False, True):                   # and with the splits' exchange giving up
+        if forced and batch > 4:
+            break
+        ctx.debug_force_merge_timeout(forced)
+        try:
+            out, aq, asc = exact_step(skv, ctx, kv, lut4096, 0, positions, qq, kq, vq, q17=True)
+        finally:
+            ctx.debug_force_merge_timeout(False)
+        for b, p in enumerate(positions):
+            if not forced:
+                scs[b].want = scs[b].step_q17(qq[b], kq[b], vq[b], p, cos[p], sin[p], fp=False, integer=True)["int"]
+            ref = scs[b].want.reshape(4096)
+            diff = np.flatnonzero(out[b] != ref)
+            assert diff.size == 0, f"seq {b} position {p}: {diff.size} Q15.17 values differ (first {diff[:4]})"
+            q14, e8 = O.a14_q17(ref.reshape(128, 32))
+            assert (asc[b] == e8).all() and (aq[b] == O.pack_a14(q14)).all(), f"seq {b}: A14"
+    kv.close()
+
+
+@pytest.mark.parametrize("batch,bias", [(1, "tail"), (32, "steep")])
+def test_exact_cost_of_rising_scores(skv, ctx, lut4096, batch, bias):
+    """Rising scores cost a small factor over random ones: 1.6 at batch 1, where one split's maxima do not fit its
+    entries, 1.8 at batch 32 (without the ordered pass 14 and 5.5).  The limit is twice the larger."""
+    _note(f"case: exact, cost of rising scores, batch {batch}, {bias}")
+    p, times = 4095, []
+    out = ctx.alloc(batch * 4096 * 4)
+    kh, vh = history(65000, p)
+    for raised in (False, True):
+        if raised:
+            kh, _ = biased_history(65000, p, BIASES[bias](p))
+        kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=p + 1)
+        for b in range(batch):
+            prefill(skv, ctx, kv, lut4096, 0, b, kh, vh, chunk=p)
+        q, k, v = (ctx.to_device(x) for x in (biased_query(65001, batch), f32_normal(65002, (batch, 4096)),
+                                              f32_normal(65003, (batch, 4096))))
+        runs = []
+        for _ in range(7):
+            ctx.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                skv.swiftkv_attention_exact(ctx, q, k, v, kv, lut4096, None, None, 0, [p] * batch, out)
+            ctx.synchronize()
+            runs.append(time.perf_counter() - t0)
+        times.append(sorted(runs)[3] / 20 * 1e6)
+        for buf in (q, k, v):
+            buf.free()
+        kv.close()
+    out.free()
+    _note(f"  {times[0]:.1f} us, rising {times[1]:.1f} us")
+    assert times[1] < 3.6 * times[0]
