@@ -777,13 +777,21 @@ __device__ __attribute__((noinline)) int32_t ordered_pass(int8_t* page, SharedPt
 // before: scores, coefficients (the new token's too), then the ordered pass
 // from `y` (Y in waves 0 and 1, Z in wave 2).  Out of line like it.
 __device__ __attribute__((noinline)) int32_t run_rest(int8_t* page, SharedPtr shared, int cap_arg, int first_arg,
-                                                      int end_arg, int32_t max_before, QueryLimbs ql, int q3, int32_t y) {
+                                                      int end_arg, int32_t max_before, v4i q0, v4i q1, v4i q2, int q3,
+                                                      int32_t y) {
     Shared& sh = *(Shared*)shared;
     const int cap = uniform(cap_arg), first = uniform(first_arg), end = uniform(end_arg), count = end - first;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int c = lane & 7, r = lane >> 3;
     const Page pg = make_page(page_rsrc(uniform(page), cap), cap, c, r);
     const int blocks = (count + kBlock - 1) / kBlock;
+    QueryLimbs ql;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        ql.w[0][j] = q0[j];
+        ql.w[1][j] = q1[j];
+        ql.w[2][j] = q2[j];
+    }
     KBlock kb;
     load_k(pg, first + wave * kBlock, wave < blocks, kb);
     for (int blk = wave; blk < blocks; blk += kWaves) {
@@ -1476,8 +1484,9 @@ __global__ __launch_bounds__(kThreads) void exact_kernel(const int8_t* layer_pag
         if (add_new) {
             const int32_t before = wave == 2 ? static_cast<int32_t>(sh.pool_z[fail_at])
                                              : sh.pool[fail_at][d & (kHeadDim - 1)];
-            y = run_rest(page_of(b, h), (SharedPtr)&sh, cap, fail_at * C, pos, sh.max_before[fail_at], ql, q3 ? 1 : 0,
-                         before);
+            auto limbs = [&](int k) { return v4i{ql.w[k][0], ql.w[k][1], ql.w[k][2], ql.w[k][3]}; };
+            y = run_rest(page_of(b, h), (SharedPtr)&sh, cap, fail_at * C, pos, sh.max_before[fail_at], limbs(0),
+                         limbs(1), limbs(2), q3 ? 1 : 0, before);
             if (wave == 2 && lane == 0) sh.z = static_cast<uint32_t>(y);
             __syncthreads();
             z = sh.z;
