@@ -12,9 +12,9 @@ bit for bit:
 
 Launches of up to 4 sequences split a head over 8, 4 or 2 workgroups (256
 tokens or more each) that exchange maxima and sums; larger ones give a
-workgroup whole heads, several in turn past 8 sequences; short sequences past 8
-take a kernel of their own.  The large-query, rescale-chain and saturation
-cases run in each."""
+workgroup whole heads, several in turn past 8 sequences; batches past 8 of short
+sequences (up to 768 tokens, or 1280 past 16 sequences) take a kernel of their
+own.  The large-query, rescale-chain and saturation cases run in each."""
 import sys
 import time
 
@@ -113,6 +113,7 @@ def test_exact_matches_reference_decode(skv, ctx, lut4096, golden, case):
     ([300, 1030, 1], "normal", False, True),   # split two ways
     ([700], "t3", False, True),                # split three ways
     ([300, 1030, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),   # whole heads, two turns
+    ([300, 767, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),    # short sequences' kernel
 ])
 def test_exact_matches_oracle_integer_recurrence(skv, ctx, lut4096, rope_tables, positions, dist, q17, big_query):
     """big_query: queries past 64.0 in some heads (and saturated channels in
@@ -202,21 +203,24 @@ def saturating_history(n, mag, lead, flip):
 
 def saturation_cases(mag, batch):
     """(position, lead, flip) per sequence: Y first saturates after 16384 / mag
-    tokens (lead 0), or at token 968, 200 tokens into its 256-token chunk (the
-    composed part there), with lead = (968 - 16384 / mag) / 2."""
+    tokens (lead 0), or at token 968, 200 tokens into the short-sequence
+    kernel's 256-token chunk (the composed part there), with lead = (968 -
+    16384 / mag) / 2.  17 sequences stay short enough for that kernel."""
     late = int(round((968 - 16384 / mag) / 2))
-    cases = [(1300, 0, 1000), (1250, late, 1100), (1100, 0, 900)]
+    cases = [(1300 if batch < 17 else 1279, 0, 1000), (1250, late, 1100), (1100, 0, 900)]
     return [cases[b % len(cases)] for b in range(batch)]
 
 
-# batch 1 and 3: split heads; 9: whole heads in turn
-@pytest.mark.parametrize("mag,batch", [(31.0, 1), (31.0, 3), (31.0, 9), (40.0, 1), (40.0, 3), (40.0, 9)])
+# batch 1 and 3: split heads; 9: whole heads in turn; 17: short sequences' kernel
+@pytest.mark.parametrize("mag,batch", [(31.0, 1), (31.0, 3), (31.0, 9), (40.0, 1), (40.0, 3), (40.0, 9),
+                                       (31.0, 17), (40.0, 17)])
 def test_exact_y_saturates(skv, ctx, lut4096, rope_tables, mag, batch):
-    """Y reaches INT32_MAX and INT32_MIN (alternate channels) early in a chunk
-    (its ordered part) or late in one (its composed part), stays, and comes
-    back: the saturating adds, the batch sums taken at once away from the
-    ends of the range, and the composed clamp-add maps, against the oracle's
-    integer recurrence bit for bit.  Shift 15 takes the fused-multiply-add
+    """Y reaches INT32_MAX and INT32_MIN (alternate channels), stays, and comes
+    back, against the oracle's integer recurrence bit for bit: sums that fail
+    their bounds and the ordered pass that takes their place, and in the
+    short-sequence kernel the saturating adds of a chunk's ordered part, the
+    batch sums taken at once away from the ends of the range, and the composed
+    clamp-add maps of its other part.  Shift 15 takes the fused-multiply-add
     term form, shift 16 the rint form."""
     _note(f"case: exact, saturating Y, |V| = {mag}, batch {batch}")
     cos, sin = rope_tables
@@ -246,17 +250,17 @@ def test_exact_y_saturates(skv, ctx, lut4096, rope_tables, mag, batch):
     kv.close()
 
 
-@pytest.mark.parametrize("seed,batch", [(99001, 1), (99004, 3), (99009, 9)])
+@pytest.mark.parametrize("seed,batch", [(99001, 1), (99004, 3), (99009, 9), (99017, 17)])   # launch forms as above
 def test_exact_y_saturates_mixed_shifts(skv, ctx, lut4096, rope_tables, seed, batch):
     """Y saturates while the V shifts change from token to token (magnitudes
-    15 to 130 per token and 1024-channel block: shifts 14 to 18), so batches
-    and composed runs switch between the fused-multiply-add, rint and integer
-    term forms around the saturation points; keys zero except a few tokens
+    15 to 130 per token and 1024-channel block: shifts 14 to 18), so blocks,
+    batches and composed runs switch between the fused-multiply-add, rint and
+    integer term forms around the saturation points; keys zero except a few tokens
     that set new maxima.  Bit for bit against the oracle's recurrence."""
     _note(f"case: exact, saturating Y with mixed shifts, seed {seed}, batch {batch}")
     cos, sin = rope_tables
     rng = np.random.default_rng(seed)
-    positions = [int(p) for p in rng.integers(500, 1400, batch)]
+    positions = [int(p) for p in rng.integers(500, 1400 if batch < 17 else 1280, batch)]
     kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=max(positions) + 1)
     scs = []
     chan_sign = np.where(np.arange(4096) % 2 == 0, 1.0, -1.0)
@@ -507,7 +511,9 @@ def check_against_oracle(skv, ctx, lut, rope_tables, positions, dist, seed, step
 
 @pytest.mark.parametrize("positions,dist", [
     ([256], "normal"),                                           # a split of the new token alone
-    ([2047, 2048], "t3"),                                        # 4 splits of 512 and 768 tokens
+    ([2047, 2048], "t3"),                                        # 3 splits of 768 tokens, as the longer one has it
+    ([2047, 2047], "t3"),                                        # 4 of 512, all full but for the new token's place
+    ([1536, 2047], "normal"),                                    # the shorter one's last split: the new token alone
     ([900], "rising"),                                           # more new maxima than a split publishes
     ([464, 464, 1100], "wide"),                                  # split heads with V shifts of 16 and more
     ([769, 0, 1, 63, 64, 65, 128, 1025, 448, 1100], "normal"),   # whole heads, two turns, one of no cached token
@@ -526,8 +532,8 @@ def test_exact_launch_forms(skv, ctx, lut4096, rope_tables, positions, dist):
 @pytest.mark.parametrize("batch", [2, 5])   # split heads, and whole ones
 def test_exact_flat_attention(skv, ctx, lut4096, rope_tables, batch):
     """Keys near zero, so every coefficient is near 1.0 and Z reaches 2,400, under V of 1, 6, 40 and 200 per
-    block of 1024 channels: sums whose bounds stay below the int32 range whole, cut at every eighth block of
-    tokens, cut at every block, and not even then (those run token by token)."""
+    block of 1024 channels: sums whose bounds stay below the int32 range whole, cut once or twice, cut at every
+    block or two, and not even then (those run token by token)."""
     _note(f"case: exact, flat attention, batch {batch}")
     cos, sin = rope_tables
     positions = [2400 - 700 * (b % 2) for b in range(batch)]
@@ -545,6 +551,8 @@ def test_exact_flat_attention(skv, ctx, lut4096, rope_tables, batch):
         ref = scs[b].step_q17(qq[b], kq[b], vq[b], p, cos[p], sin[p], fp=False, integer=True)["int"].reshape(4096)
         diff = np.flatnonzero(out[b] != ref)
         assert diff.size == 0, f"seq {b} position {p}: {diff.size} Q15.17 values differ (first {diff[:4]})"
+        q14, e8 = O.a14_q17(ref.reshape(128, 32))
+        assert (asc[b] == e8).all() and (aq[b] == O.pack_a14(q14)).all(), f"seq {b}: A14"
     kv.close()
 
 

@@ -479,3 +479,33 @@ def test_oracle_step_matches_reference_build_long_context(oracle, rope_tables):
         kc, ks, vc, vs = rc.row(h, pos)
         assert (kc == sc.kc[h, pos]).all() and (ks == sc.ks[h, pos]).all()
         assert (vc == sc.vc[h, pos]).all() and (vs == sc.vs[h, pos]).all()
+
+
+def test_exp_in_doubles_equals_the_rule(oracle):
+    """The device's exp takes round-half-even of x log2(e) from a double product and drops the rule's special
+    cases; written out here the same way it equals the oracle's rule for every x in [-40.0, 0], where all results
+    but 0 lie, and for samples below (the device code itself is checked through the integer step)."""
+    lut = np.array([int(round(2.0 ** (30 + i / 32))) for i in range(33)], np.int64)
+
+    def interpolated(l):
+        f = l & 0x1FFFF
+        base, nxt = lut[f >> 12], lut[(f >> 12) + 1]
+        interp = base + (((nxt - base) * (f & 0xFFF) + (1 << 11)) >> 12)
+        sh = 13 - (l >> 17)
+        return np.where(sh < 32, (interp + (1 << ((sh - 1) & 31))) >> (sh & 31), 0)
+
+    def device_form(x):
+        l = np.clip(np.rint(x.astype(np.float64) * (3025551.0 * 2.0 ** -21)), -2.0 ** 31, 2.0 ** 31 - 1)
+        return interpolated(l.astype(np.int64))
+
+    def rule(x):   # 64-bit integers, as the oracle has it
+        p = x.astype(np.int64) * 3025551
+        l = (p + (1 << 20) - 1 + ((p >> 21) & 1)) >> 21
+        return np.where(x >= 0, 1 << 17, np.where(x <= -(32 << 17), 0, interpolated(np.maximum(l, -(1 << 23)))))
+
+    x = np.arange(-(40 << 17), 1, dtype=np.int32)
+    assert (device_form(x) == rule(x)).all()
+    far = np.concatenate([-np.logspace(np.log10(40 << 17), np.log10(2.0 ** 31), 5000).astype(np.int64), [-2 ** 31]])
+    assert (device_form(far) == 0).all()
+    near = np.concatenate([x[-3000:], x[::997], np.arange(-(32 << 17) - 300, -(32 << 17) + 300), far[far >= -2 ** 31]])
+    assert (rule(near) == np.array([oracle.exp_neg_q17(int(v)) for v in near])).all()
