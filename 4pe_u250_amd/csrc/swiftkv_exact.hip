@@ -170,9 +170,11 @@ struct Shared {
     int32_t stage[kStageRows][kHeadDim];
     __attribute__((aligned(16))) int32_t stage_z[kStageRows];
     // The ordered pass: its rows (tokens, or stretches as kSumRow | index), and
-    // per staged row the bounds of a stretch's sum.
+    // per half of the staging rows the largest bounds of its sums (kNoBound
+    // without any) and whether it holds a special token.
     uint16_t order[kExactMaxTokens + kMaxBlocks + 8];
-    __attribute__((aligned(16))) float stage_b[kStageRows][kGroupsPerHead];
+    float round_bound[2][kGroupsPerHead];
+    uint32_t round_special[2];
     uint32_t staged;                              // rows taken so far
     uint32_t unbounded;                           // a sum could saturate Y
     // Special (first or rescaling) tokens of a split that cannot fold its own
@@ -588,10 +590,11 @@ __device__ __forceinline__ int32_t run_round(const Shared& sh, int at, int d, in
     };
     const int own = static_cast<int>(sh.stage_mult[at + lane]);   // of row `lane`
     const int own_z = Z ? sh.stage_z[at + lane] : 0;
-    const float own_bound = sh.stage_b[at + lane][0];
+    const uint32_t has_special = sh.round_special[at / kRound];
+    const float bound = Z ? kNoBound : sh.round_bound[at / kRound][g];
     load(0);
-    const bool special = __builtin_amdgcn_ballot_w64(own != __float_as_int(1.0f)) != 0u;
-    const uint64_t sums = Z ? 0u : __builtin_amdgcn_ballot_w64(own_bound != kNoBound);
+    const bool special = uniform(has_special) != 0u;
+    const bool sums = uniform(__float_as_int(bound)) != __float_as_int(kNoBound);
     load(kRound / 2);
     auto term = [&](int j) { return Z ? __builtin_amdgcn_readlane(own_z, j) : x[j]; };
     auto step = [&](int j) {
@@ -601,15 +604,13 @@ __device__ __forceinline__ int32_t run_round(const Shared& sh, int at, int d, in
     };
     if (Z && !special) {   // Z stays below 2^30: a sum in any order
         y += __builtin_amdgcn_readlane(static_cast<int>(wave_scan_add(static_cast<uint32_t>(own_z))), 63);
-    } else if (sums == 0u && !special) {
+    } else if (!sums && !special) {
 #pragma unroll
         for (int j = 0; j < kRound; ++j) y = __builtin_elementwise_add_sat(y, term(j));
-    } else if (sums == 0u) {
+    } else if (!sums) {
 #pragma unroll
         for (int j = 0; j < kRound; ++j) step(j);
     } else {
-        float bound = kNoBound;
-        for (uint64_t s = sums; s != 0u; s &= s - 1ull) bound = fmaxf(bound, sh.stage_b[at + __builtin_ctzll(s)][g]);
         int32_t hi = y, lo = y;
 #pragma unroll
         for (int j = 0; j < kRound; ++j) {
@@ -742,14 +743,25 @@ __device__ __attribute__((noinline)) int32_t ordered_pass(int8_t* page, SharedPt
             const float coef = __builtin_fabsf(__uint_as_float(x));
             float mult = special ? coef * 0x1p-17f : 1.0f;   // 0.0 for the sequence's first token
             int32_t z = special ? 1 << 17 : static_cast<int32_t>(coef);
-            float4 bound = make_float4(kNoBound, kNoBound, kNoBound, kNoBound);
+            float4 bound = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (sum && !past) {
                 z = static_cast<int32_t>(sh.pool_z[row & (kSumRow - 1)]);
                 bound = *reinterpret_cast<const float4*>(sh.pool_b[row & (kSumRow - 1)]);
             }
             sh.stage_mult[at] = __float_as_uint(mult);
             sh.stage_z[at] = z;
-            *reinterpret_cast<float4*>(sh.stage_b[at]) = bound;
+            const uint64_t specials = __builtin_amdgcn_ballot_w64(special);
+            if (pieces) {                         // the bounds are not negative: their bits compare as integers do
+                const float b[kGroupsPerHead] = {bound.x, bound.y, bound.z, bound.w};
+#pragma unroll
+                for (int g = 0; g < kGroupsPerHead; ++g) {
+                    const int32_t most = wave_scan_max(sum && !past ? __float_as_int(b[g]) : __float_as_int(kNoBound));
+                    if (lane == 63) sh.round_bound[round & 1][g] = __int_as_float(most);
+                }
+            } else if (lane < kGroupsPerHead) {
+                sh.round_bound[round & 1][lane] = kNoBound;
+            }
+            if (lane == 0) sh.round_special[round & 1] = specials != 0u;
         };
         describe(0);
         for (int b = 0; b < barriers; ++b) {
