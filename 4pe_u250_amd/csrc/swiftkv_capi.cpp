@@ -618,16 +618,21 @@ int32_t exact_split(int32_t max_pos, int32_t batch) {
     return std::min((tokens + kSplitQuantum - 1) / kSplitQuantum * kSplitQuantum, kExactMaxTokens);
 }
 
-// Which kernel an integer-compatibility launch runs: batches past 8 rows whose
-// longest sequence is short take the one with four workgroups per CU (whose
-// turns hide each other's latencies), the rest the one that sums in any order
-// (one workgroup per CU).  Context 512 / 1024 / 2048, us, short kernel against
-// the other: batch 9 27.5 / 42.5 / 72.2 against 29.2 / 39.7 / 57.6; batch 16
-// 30.6 / 48.1 / 78.3 against 33.8 / 44.2 / 65.8; batch 24 35.4 / 57.0 / 97.9
-// against 45.0 / 59.7 / 92.5; batch 64 74.6 / 127.0 / 226.6 against 99.1 /
-// 135.6 / 217.0.  Up to 8 rows (one turn per workgroup) the other kernel is
-// ahead at every context.
-bool exact_is_short(int32_t max_pos, int32_t batch) { return batch > 8 && max_pos + 1 <= (batch <= 16 ? 768 : 1280); }
+// Which kernel an integer-compatibility launch runs: where the longest sequence
+// is short, the one with four workgroups per CU (whose turns hide each other's
+// latencies, and whose chain of barriers is shorter), else the one that sums in
+// any order (one workgroup per CU).  Context 512 / 1024 / 2048, us, short kernel
+// against the other: batch 9 26.9 / 39.9 / 63.5 against 27.9 / 40.1 / 54.9;
+// batch 16 29.1 / 41.1 / 74.3 against 31.1 / 41.5 / 59.9; batch 24 33.4 / 49.7 /
+// 96.0 against 42.1 / 56.0 / 87.1; batch 64 64.9 / 122.1 / 223.1 against 99.6 /
+// 135.2 / 212.8 (context 1536 73.4 against 72.2 at batch 24, 172.1 against 172.9
+// at 64).  Up to 8 rows (one turn per workgroup) context 2 / 64 / 129 / 144 / 192:
+// batch 1 7.2 / 10.5 / 12.4 / 12.4 / 13.6 against 8.6 / 11.6 / 13.2 / 13.3 / 13.4,
+// batch 4 7.3 / 11.3 / 13.1 / 14.4 / 14.9 against 8.7 / 12.0 / 13.6 / 13.7 / 13.8,
+// batch 8 7.3 / 11.5 / 13.5 / 14.4 / 15.8 against 8.8 / 12.1 / 14.5 / 14.7 / 14.8.
+bool exact_is_short(int32_t max_pos, int32_t batch) {
+    return max_pos + 1 <= (batch <= 8 ? 136 : batch <= 16 ? 768 : 1280);
+}
 
 int run_exact(swiftkv_context* ctx, const void* q, const void* k, const void* v, StepInput in,
               swiftkv_kv_cache* kv, const swiftkv_rope_lut* lut, uint8_t* act_q, uint8_t* act_scale,

@@ -1,5 +1,5 @@
-// swiftkv_exact_short.hip -- the integer-compatibility step for batches of
-// short sequences: one 4-wave workgroup per (sequence, head), four to a CU, so
+// swiftkv_exact_short.hip -- the integer-compatibility step for short
+// sequences: one 4-wave workgroup per (sequence, head), four to a CU, so
 // that one's latencies hide behind the others'.  swiftkv_exact.hip's kernel
 // (one 8-wave workgroup per CU, sums in any order) pays about 6 us per head for
 // its exchange of maxima, its fold and its epilogue; this one takes chunks of

@@ -12,9 +12,8 @@ bit for bit:
 
 Launches of up to 4 sequences split a head over 8, 4 or 2 workgroups (256
 tokens or more each) that exchange maxima and sums; larger ones give a
-workgroup whole heads, several in turn past 8 sequences; batches past 8 of short
-sequences (up to 768 tokens, or 1280 past 16 sequences) take a kernel of their
-own.  The large-query, rescale-chain and saturation cases run in each."""
+workgroup whole heads, several in turn past 8 sequences; short sequences (up to
+136 tokens to 8 sequences, 768 to 16, 1280 beyond) take a kernel of their own.  The large-query, rescale-chain and saturation cases run in each."""
 import sys
 import time
 
@@ -519,7 +518,11 @@ def check_against_oracle(skv, ctx, lut, rope_tables, positions, dist, seed, step
     ([769, 0, 1, 63, 64, 65, 128, 1025, 448, 1100], "normal"),   # whole heads, two turns, one of no cached token
     ([800, 511, 1000, 64, 900, 700, 1, 300, 769], "wide"),       # V shifts up to 25, in every term form
     ([1000] * 9, "rising"),                                      # more accumulators than a workgroup holds
-    ([767, 0, 255, 256, 257, 511, 512, 1, 64], "normal"),        # the kernel for short sequences, at its bound
+    ([767, 0, 255, 256, 257, 511, 512, 1, 64], "normal"),        # the kernel for short sequences, at its bounds
+    ([135], "wide"),
+    ([136], "wide"),
+    ([135, 0, 64, 1, 63, 100, 127, 65], "t3"),
+    ([136, 0, 64, 1, 63, 100, 127, 65], "t3"),
     ([1279] + [40] * 16, "t3"),
     ([1280] + [40] * 16, "t3"),
 ])
