@@ -67,6 +67,7 @@ _SIGNATURES = {
     "swiftkv_synchronize": (C.c_int, [_vp]),
     "swiftkv_set_split_tokens": (C.c_int, [_vp, _i32]),
     "swiftkv_debug_set_split_generation": (C.c_int, [_vp, C.c_uint32, _i32]),
+    "swiftkv_debug_exact_plan": (C.c_int, [_i32, _vp, _i32, C.POINTER(_i32), C.POINTER(_i32)]),
     "swiftkv_debug_exchange_words": (C.c_int, [_vp, C.POINTER(C.c_int64)]),
     "swiftkv_debug_force_merge_timeout": (C.c_int, [_vp, _i32]),
     "swiftkv_debug_set_step_shape": (C.c_int, [_vp, _i32, _i32]),
@@ -522,6 +523,16 @@ def step_plan(positions, cus: int = 256, workgroups_per_cu: int = 3, split_token
                                          int(pos.size), C.byref(split), C.byref(grid), C.byref(waves),
                                          C.byref(block), _host_ptr(rows)))
     return split.value, grid.value, waves.value, block.value, rows
+
+
+def exact_plan(positions, cus: int = 256):
+    """The plan of one launch of the integer-compatibility step (host-only, no
+    device needed): (whether it runs the kernel for short sequences, splits of
+    the longest sequence)."""
+    pos = np.ascontiguousarray(np.atleast_1d(np.asarray(positions, dtype=np.int32)))
+    short, splits = C.c_int32(), C.c_int32()
+    _check(lib().swiftkv_debug_exact_plan(int(cus), _host_ptr(pos), int(pos.size), C.byref(short), C.byref(splits)))
+    return bool(short.value), splits.value
 
 
 def swiftkv_attention_noalloc(ctx: Context, q, k, v, kv_cache: KVCache, rope_lut: RopeLut,

@@ -618,20 +618,43 @@ int32_t exact_split(int32_t max_pos, int32_t batch) {
     return std::min((tokens + kSplitQuantum - 1) / kSplitQuantum * kSplitQuantum, kExactMaxTokens);
 }
 
-// Which kernel an integer-compatibility launch runs: where the longest sequence
-// is short, the one with four workgroups per CU (whose turns hide each other's
-// latencies, and whose chain of barriers is shorter), else the one that sums in
-// any order (one workgroup per CU).  Context 512 / 1024 / 2048, us, short kernel
-// against the other: batch 9 26.9 / 39.9 / 63.5 against 27.9 / 40.1 / 54.9;
-// batch 16 29.1 / 41.1 / 74.3 against 31.1 / 41.5 / 59.9; batch 24 33.4 / 49.7 /
-// 96.0 against 42.1 / 56.0 / 87.1; batch 64 64.9 / 122.1 / 223.1 against 99.6 /
-// 135.2 / 212.8 (context 1536 73.4 against 72.2 at batch 24, 172.1 against 172.9
-// at 64).  Up to 8 rows (one turn per workgroup) context 2 / 64 / 129 / 144 / 192:
-// batch 1 7.2 / 10.5 / 12.4 / 12.4 / 13.6 against 8.6 / 11.6 / 13.2 / 13.3 / 13.4,
-// batch 4 7.3 / 11.3 / 13.1 / 14.4 / 14.9 against 8.7 / 12.0 / 13.6 / 13.7 / 13.8,
-// batch 8 7.3 / 11.5 / 13.5 / 14.4 / 15.8 against 8.8 / 12.1 / 14.5 / 14.7 / 14.8.
-bool exact_is_short(int32_t max_pos, int32_t batch) {
-    return max_pos + 1 <= (batch <= 8 ? 136 : batch <= 16 ? 768 : 1280);
+// Which kernel an integer-compatibility launch runs (a.rows is set): the one
+// that sums in any order, a workgroup per CU taking heads in turn, or the one for
+// short sequences, four workgroups to a CU, whose chain of barriers is shorter
+// and whose latencies hide behind each other, but whose cost per token is higher.
+//
+// Where every head has a CU of its own the line lies by context: 2 / 64 / 129 /
+// 144 / 192 tokens, us, short kernel against the other: batch 1 7.2 / 10.5 /
+// 12.4 / 12.4 / 13.6 against 8.6 / 11.6 / 13.2 / 13.3 / 13.4, batch 4 7.3 / 11.3 /
+// 13.1 / 14.4 / 14.9 against 8.7 / 12.0 / 13.6 / 13.7 / 13.8, batch 8 7.3 / 11.5 /
+// 13.5 / 14.4 / 15.8 against 8.8 / 12.1 / 14.5 / 14.7 / 14.8.
+//
+// Past that by what each is expected to take, us: the other 7.0 and 0.0103 a
+// token for each head a workgroup takes; the short one the chain of the longest
+// sequence, 14 and 0.0215 a token, or, where more, what the CUs do in all, 0.8
+// and 0.0136 a token for each head.  Batches of one length cross where the
+// measured times do: context 512 / 1024 / 2048 batch 9 26.9 / 39.9 / 63.5 against
+// 27.9 / 40.1 / 54.9; 16 29.1 / 41.1 / 74.3 against 31.1 / 41.5 / 59.9; 24 33.4 /
+// 49.7 / 96.0 against 42.1 / 56.0 / 87.1; 64 64.9 / 122.1 / 223.1 against 99.6 /
+// 135.2 / 212.8.  Mixed lengths: 63 of 100 and one of 1300 43 against 87, one of
+// 3000 and 63 of 64 77 against 98, two of 4095 and 254 of 30 100 against 282, 16
+// to 64 of up to 2424 tokens 145 against 163; but one of 1400 and 23 of 100 45
+// against 41, one of 2500 and 31 of 20 64 against 55, one of 800 and 8 of 50 31
+// against 20.
+bool exact_is_short(const StepArgs& a, int32_t cus) {
+    const int32_t turn = std::max(cus / kHeads, 1);   // rows that have a CU per head
+    const int32_t longest = static_cast<int32_t>(a.rows[0] >> 8) + 1;
+    if (a.batch <= turn) return longest <= 136;
+    float load[kMaxBatchPerLaunch] = {}, all = 0.0f, most = 0.0f;
+    for (int32_t z = 0; z < a.batch; ++z) {
+        const float len = static_cast<float>((a.rows[z] >> 8) + 1u);
+        const int32_t slot = (z / turn) % 2 == 0 ? z % turn : turn - 1 - z % turn;   // as launch_exact deals them
+        load[slot] += 7.0f + 0.0103f * len;
+        most = std::max(most, load[slot]);
+        all += 0.8f + 0.0136f * len;
+    }
+    const float together = 4.0f + all * kHeads / static_cast<float>(cus);
+    return std::max(14.0f + 0.0215f * static_cast<float>(longest), together) < 0.92f * (4.0f + most);
 }
 
 int run_exact(swiftkv_context* ctx, const void* q, const void* k, const void* v, StepInput in,
@@ -668,7 +691,7 @@ int run_exact(swiftkv_context* ctx, const void* q, const void* k, const void* v,
         a.merge_polls = ctx->merge_fault_test ? 1u : kMergePolls;
         a.merge_tag_skew = ctx->merge_fault_test ? 1u : 0u;
         ProfilePair* p = profile_begin(ctx, SWIFTKV_KERNEL_EXACT);
-        SKV_HIP(exact_is_short(max_pos, nb) ? launch_exact_short(a, in.format == kInQ17, ctx->stream)
+        SKV_HIP(exact_is_short(a, ctx->cus) ? launch_exact_short(a, in.format == kInQ17, ctx->stream)
                                             : launch_exact(a, grid_splits, ctx->cus, in.format == kInQ17, ctx->stream));
         profile_end(ctx, p);
     }
@@ -917,6 +940,27 @@ int swiftkv_debug_step_plan(int32_t cus, int32_t workgroups_per_cu, int32_t spli
     if (out_block_tokens) *out_block_tokens = shape.block_tokens;
     if (out_rows)
         for (int32_t z = 0; z < batch; ++z) out_rows[z] = static_cast<int32_t>(a.rows[z] & 0xffu);
+    return ok();
+}
+
+int swiftkv_debug_exact_plan(int32_t cus, const int32_t* positions, int32_t batch, int32_t* out_short,
+                             int32_t* out_splits) {
+    if (!positions || !out_short || !out_splits) return fail(SWIFTKV_EINVAL, "null argument");
+    if (cus < 1) return fail(SWIFTKV_EINVAL, "cus %d must be positive", cus);
+    if (batch < 1 || batch > kMaxBatchPerLaunch)
+        return fail(SWIFTKV_ERANGE, "batch %d outside [1, %d] (one launch)", batch, kMaxBatchPerLaunch);
+    int32_t max_pos = 0;
+    for (int32_t b = 0; b < batch; ++b) {
+        if (positions[b] < 0 || positions[b] >= kExactMaxTokens)
+            return fail(SWIFTKV_ERANGE, "position %d outside [0, %d)", positions[b], kExactMaxTokens);
+        max_pos = std::max(max_pos, positions[b]);
+    }
+    StepArgs a;
+    a.batch = batch;
+    set_rows(a, positions);
+    *out_short = exact_is_short(a, cus);
+    const int32_t split = exact_split(max_pos, batch);
+    *out_splits = *out_short ? 1 : (max_pos + split) / split;
     return ok();
 }
 

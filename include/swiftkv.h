@@ -125,6 +125,11 @@ int swiftkv_debug_set_step_shape(swiftkv_context* ctx, int32_t waves, int32_t bl
 int swiftkv_debug_step_plan(int32_t cus, int32_t workgroups_per_cu, int32_t split_tokens, const int32_t* positions,
                             int32_t batch, int32_t* out_split_tokens, int32_t* out_grid_splits, int32_t* out_waves,
                             int32_t* out_block_tokens, int32_t* out_rows);
+/* Testing aid with no counterpart in the reference: the same for one launch of
+ * the integer-compatibility entry: whether it runs the kernel for short
+ * sequences, and the splits of its longest sequence. */
+int swiftkv_debug_exact_plan(int32_t cus, const int32_t* positions, int32_t batch, int32_t* out_short,
+                             int32_t* out_splits);
 /* Testing aid with no counterpart in the reference.  A head split across
  * workgroups is merged inside the launch through 64-bit words tagged with the
  * (sequence row, head)'s generation + 1, which every launch that merges the

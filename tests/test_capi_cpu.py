@@ -176,6 +176,28 @@ def test_step_plan(skv, positions, split, want):
     assert got[:4] == want
 
 
+@pytest.mark.parametrize("positions,short,splits", [
+    ([135], True, 1), ([136], False, 1), ([135] * 8, True, 1), ([136] + [0] * 7, False, 1),   # a CU per head
+    ([4095], False, 8), ([1300], False, 6), ([4095] * 2, False, 4), ([2047] * 4, False, 2), ([4095] * 5, False, 1),
+    ([511] * 9, True, 1), ([2047] * 9, False, 1), ([511] * 16, True, 1), ([2047] * 16, False, 1),
+    ([1023] * 24, True, 1), ([2047] * 24, False, 1), ([1023] * 64, True, 1), ([2047] * 64, False, 1),
+    ([1300] + [100] * 63, True, 1),      # one long sequence does not decide for a batch of short ones
+    ([3000] + [64] * 63, True, 1), ([4095] * 2 + [30] * 254, True, 1),
+    ([1400] + [100] * 23, False, 1),     # unless its chain is what they would wait for
+    ([800] + [50] * 8, False, 1), ([2500] + [20] * 31, False, 1),
+])
+def test_exact_plan(skv, positions, short, splits):
+    """The kernel that measured faster, and the splits of the longest sequence."""
+    assert skv.exact_plan(positions) == (short, splits)
+    assert skv.exact_plan(positions[::-1]) == (short, splits)
+
+
+def test_exact_plan_refuses(skv):
+    for positions, cus in (([4096], 256), ([-1], 256), ([0] * 257, 256), ([0], 0)):
+        with pytest.raises(skv.SwiftKVError):
+            skv.exact_plan(positions, cus)
+
+
 def test_step_plan_orders_rows_longest_first(skv):
     split, grid, waves, block, rows = skv.step_plan([5, 100, 100, 3, 4095, 0, 100])
     assert rows.tolist() == [4, 1, 2, 6, 0, 3, 5]       # equal positions keep sequence order

@@ -12,8 +12,9 @@ bit for bit:
 
 Launches of up to 4 sequences split a head over 8, 4 or 2 workgroups (256
 tokens or more each) that exchange maxima and sums; larger ones give a
-workgroup whole heads, several in turn past 8 sequences; short sequences (up to
-136 tokens to 8 sequences, 768 to 16, 1280 beyond) take a kernel of their own.  The large-query, rescale-chain and saturation cases run in each."""
+workgroup whole heads, several in turn past 8 sequences; launches of short
+sequences take a kernel of their own (exact_plan says which).  The large-query,
+rescale-chain and saturation cases run in each."""
 import sys
 import time
 
@@ -112,7 +113,7 @@ def test_exact_matches_reference_decode(skv, ctx, lut4096, golden, case):
     ([300, 1030, 1], "normal", False, True),   # split two ways
     ([700], "t3", False, True),                # split three ways
     ([300, 1030, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),   # whole heads, two turns
-    ([300, 767, 1, 700, 5, 257, 256, 511, 64], "normal", False, True),    # short sequences' kernel
+    ([300, 257, 256, 255, 1, 64, 290, 310] * 3, "normal", False, True),   # short sequences' kernel
 ])
 def test_exact_matches_oracle_integer_recurrence(skv, ctx, lut4096, rope_tables, positions, dist, q17, big_query):
     """big_query: queries past 64.0 in some heads (and saturated channels in
@@ -225,6 +226,7 @@ def test_exact_y_saturates(skv, ctx, lut4096, rope_tables, mag, batch):
     cos, sin = rope_tables
     cases = saturation_cases(mag, batch)
     positions = [c[0] for c in cases]
+    assert skv.exact_plan(positions)[0] == (batch == 17)
     kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=max(positions) + 1)
     scs = []
     for b, (p, lead, flip) in enumerate(cases):
@@ -260,6 +262,7 @@ def test_exact_y_saturates_mixed_shifts(skv, ctx, lut4096, rope_tables, seed, ba
     cos, sin = rope_tables
     rng = np.random.default_rng(seed)
     positions = [int(p) for p in rng.integers(500, 1400 if batch < 17 else 1280, batch)]
+    assert skv.exact_plan(positions)[0] == (batch == 17)
     kv = skv.KVCache(ctx, layers=1, max_batch=batch, max_seq_len=max(positions) + 1)
     scs = []
     chan_sign = np.where(np.arange(4096) % 2 == 0, 1.0, -1.0)
@@ -517,11 +520,10 @@ def check_against_oracle(skv, ctx, lut, rope_tables, positions, dist, seed, step
     ([464, 464, 1100], "wide"),                                  # split heads with V shifts of 16 and more
     ([769, 0, 1, 63, 64, 65, 128, 1025, 448, 1100], "normal"),   # whole heads, two turns, one of no cached token
     ([800, 511, 1000, 64, 900, 700, 1, 300, 769], "wide"),       # V shifts up to 25, in every term form
-    ([1000] * 9, "rising"),                                      # more accumulators than a workgroup holds
-    ([767, 0, 255, 256, 257, 511, 512, 1, 64], "normal"),        # the kernel for short sequences, at its bounds
-    ([135], "wide"),
+    ([1000] * 9, "rising"),                                      # almost every token a new maximum: short kernel,
+    ([1000] * 5, "rising"),                                      # whole heads
+    ([767, 0, 255, 256, 257, 511, 512, 1, 64], "normal"),
     ([136], "wide"),
-    ([135, 0, 64, 1, 63, 100, 127, 65], "t3"),
     ([136, 0, 64, 1, 63, 100, 127, 65], "t3"),
     ([1279] + [40] * 16, "t3"),
     ([1280] + [40] * 16, "t3"),
@@ -530,6 +532,20 @@ def test_exact_launch_forms(skv, ctx, lut4096, rope_tables, positions, dist):
     """Each way a launch is cut up, at the edges of blocks, splits, turns and the rule between the two kernels."""
     _note(f"case: exact launch forms, positions {positions}, {dist}")
     check_against_oracle(skv, ctx, lut4096, rope_tables, positions, dist, 61000 + positions[0])
+
+
+@pytest.mark.parametrize("positions,dist", [
+    ([135], "wide"),
+    ([135, 0, 64, 1, 63, 100, 127, 65], "t3"),
+    ([767, 768, 512, 511, 513, 640, 750, 560, 257] * 3, "normal"),   # past one chunk of 256 tokens, and two
+    ([256, 255, 257, 0, 1, 511, 512, 513] * 2 + [300], "wide"),
+    ([1300] + [100, 0, 256, 31] * 10, "normal"),                 # one long sequence among short ones
+])
+def test_exact_short_sequences(skv, ctx, lut4096, rope_tables, positions, dist):
+    """The kernel for short sequences at the edges of its chunks and of the rule that picks it."""
+    _note(f"case: exact, short sequences, positions {positions}, {dist}")
+    assert skv.exact_plan(positions)[0]
+    check_against_oracle(skv, ctx, lut4096, rope_tables, positions, dist, 61500 + positions[0])
 
 
 @pytest.mark.parametrize("batch", [2, 5])   # split heads, and whole ones
