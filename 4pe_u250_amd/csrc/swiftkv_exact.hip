@@ -57,16 +57,16 @@
 // buffers, context 4096, N(0, 1), us per call, the chunked kernel it replaced (Y
 // in token order through LDS, up to four workgroups per head each scoring every
 // token) against this one:
-//   batch     1           2           4           8          16          32         64
-//   normal    90.7 / 23.7 93.7 / 26.8 87.4 / 36.7 112 / 55.0 134 / 103   230 / 196  431 / 379
+//   batch     1            2            4            8            16           32           64
+//   normal    90.6 / 23.8  93.4 / 26.7  87.5 / 36.9  113 / 55.3   135 / 104    233 / 197    433 / 380
 //   scores that rise by 8 sigma over the last 200 tokens:
-//             103 / 36.3  109 / 46.5  100 / 71.6  121 / 59.4 145 / 111   239 / 214  442 / 411
+//             103 / 35.0   108 / 45.4   100 / 69.5   123 / 59.9   146 / 112    241 / 215    446 / 413
 //   every token a new maximum:
-//             556 / 114   558 / 118   518 / 129   543 / 139  583 / 269   633 / 535  1242 / 1043
+//             557 / 115    557 / 119    517 / 128    542 / 140    582 / 271    632 / 535    1243 / 1042
 // Slower than that kernel, which took every token from LDS at one rate: Y that
-// saturates for thousands of tokens, from batch 16 on (140 / 189; 435 / 717 at
-// 64), and scores that drift by 16 sigma and more over the context, from batch
-// 32 on (458 / 485 at 64; 271 / 319 at 64 and context 2048).
+// saturates for thousands of tokens, from batch 16 on (141 / 188, at 64 439 / 709),
+// and scores that drift by 16 sigma and more over the context, from batch 32 on
+// (462 / 483 at 64; 272 / 318 at 64 and context 2048).
 // Tried: two 8-wave workgroups per CU (128 registers, 480 at batch 64: their
 // streams get in each other's way, and a batch-1 launch then doubles workgroups
 // up on half the CUs, 39 against 28);
